@@ -733,10 +733,10 @@ def main():
     default_workload = m == 64 and args.nside == 1024 and dim == 16
     # the committed counter summaries profile the FP64-rerank training pass
     if h["roofline"] is not None and default_workload and args.arithmetic == "fp64":
-        tr = profile_figure("som_epoch_64x64_d16_hbm_traffic.md", "traffic_bytes_per_launch", "bmu_bf16_kernel")
+        tr = profile_figure("som_epoch_64x64_d16_hbm_traffic.md", "traffic_bytes_per_launch", "bmu_f16_kernel")
         h["roofline"]["traffic"] = None if tr is None else int(tr)
         h["roofline"]["mfma_busy"] = profile_figure("som_epoch_64x64_d16_counters.md", "mfma_busy",
-                                                    "bmu_bf16_kernel")
+                                                    "bmu_f16_kernel")
     out = {
         "metric": METRIC,
         "value": round(h["samples_per_s"], 1),
@@ -748,11 +748,11 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "bf16",
+        "dtype": "fp16",
         "data": "synthetic",
         "config": {"workload": f"batch SOM epoch, {m}x{m} hexagonal, dim {dim}, N={N} (HEALPix nside "
                                f"{args.nside}), sigma0={sigma0:g}, timed epochs of the {E}-epoch schedule from "
-                               f"init_rand(0); BF16 MFMA distance GEMM + {args.arithmetic} rerank",
+                               f"init_rand(0); FP16 MFMA distance GEMM + {args.arithmetic} rerank",
                    "map": f"{m}x{m}", "dim": dim, "samples": N, "precision": "bf16_rerank",
                    "rerank_arithmetic": args.arithmetic, "epochs_schedule": E},
         "roofline": h["roofline"],
@@ -786,8 +786,8 @@ def main():
         r3 = w3["res"]
         if r3[head_name].get("roofline") and args.arithmetic == "fp64":
             r3[head_name]["roofline"]["mfma_busy"] = profile_figure("som_epoch_100x100_d32_counters.md", "mfma_busy",
-                                                                    "bmu_bf16_kernel")
-            tr3 = profile_figure("som_epoch_100x100_d32_hbm_traffic.md", "traffic_bytes_per_launch", "bmu_bf16_kernel")
+                                                                    "bmu_f16_kernel")
+            tr3 = profile_figure("som_epoch_100x100_d32_hbm_traffic.md", "traffic_bytes_per_launch", "bmu_f16_kernel")
             r3[head_name]["roofline"]["traffic"] = None if tr3 is None else int(tr3)
         out["c3"] = {"workload": f"batch SOM epoch, 100x100 hexagonal, dim 32, N={X3.shape[0]} (HEALPix nside 2048, "
                                  "16 lognormal + 14 Gaussian + 2 angular), sigma0=50, timed epochs of the 10-epoch "

@@ -41,7 +41,7 @@ inline int check_prec(int precision, int arithmetic)
     return SOMHIP_OK;
 }
 
-// Slot order of the BF16 path.
+// Slot order of the 16-bit search.
 //
 // Base order: slot p -> neuron (p*S) mod mn, S coprime to mn and chosen so that no multiple k*S
 // (k < KSPREAD) lands on a grid neighbour offset (+-1, +-n, +-n+-1): a neuron and its grid
@@ -401,6 +401,28 @@ bool closed_form_grid(const T *topo, int m, int n, int topology)
 }
 
 // The model's weights and topography in T: float for float32 models, double for float64 models.
+// Buffers of the 16-bit search (weights of `wsize` bytes per value) and its slot order.
+hipError_t alloc_search(somhip_model *M, size_t wsize)
+{
+    const PermLayout layout = make_perm(M->m, M->n);
+    M->pblk = layout.pblk;
+    M->pblk_a = layout.pblk_a;
+    M->kpad = M->dim <= 16 ? 16 : M->dim <= 32 ? 32 : 64;
+    const size_t slots = (size_t)M->pblk * 32;
+    hipError_t e;
+    if ((e = hipMalloc((void **)&M->centre, sizeof(float) * M->kpad)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->basis, sizeof(double) * M->kpad * M->kpad)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->rot, sizeof(float) * M->kpad * 64)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->plan, sizeof(BmuPlan))) != hipSuccess ||
+        (e = hipMalloc((void **)&M->wrot, sizeof(float) * slots * M->kpad)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->norms, sizeof(double) * slots)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->frag_h, sizeof(_Float16) * slots * 16 * f16_max_nk(M->kpad))) != hipSuccess ||
+        (e = hipMalloc(&M->wslot, wsize * slots * M->kpad)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->perm, sizeof(int) * slots)) != hipSuccess)
+        return e;
+    return hipMemcpy(M->perm, layout.perm.data(), sizeof(int) * slots, hipMemcpyHostToDevice);
+}
+
 template <class T> T *model_w(somhip_model *M);
 template <> float *model_w<float>(somhip_model *M) { return M->w; }
 template <> double *model_w<double>(somhip_model *M) { return M->w64; }
@@ -409,7 +431,7 @@ template <> const float *model_topo<float>(const somhip_model *M) { return M->to
 template <> const double *model_topo<double>(const somhip_model *M) { return M->topo64; }
 
 // The BMU search: FP32 rows with the requested precision and arithmetic, FP64 rows (float64 models)
-// with the exact FP64 scan.
+// with the exact FP64 distance (after the 16-bit search).
 int search(somhip_model *M, const float *x, int64_t n, int precision, int arithmetic, int need_c2, int default_index,
            int32_t *c1, int32_t *c2, double *d1)
 {
@@ -492,7 +514,7 @@ int epoch_update_t(somhip_accum *A, int64_t cur_epoch, int64_t n_epochs, double 
         return SOMHIP_ERR_ARG;
     }
     const double sigma = epoch_sigma(sigma0, cur_epoch, n_epochs);
-    M->prepared = false;  // the derived data of the FP32 search follow the new weights
+    M->weights_changed();
     int rc;
     TimerScope ts(M->ctx, TK_UPDATE);
     if (M->separable && somhip_update_separable_fits(M->m, M->n, M->dim)) {
@@ -545,7 +567,7 @@ int iter_update_t(somhip_accum *A, T *history_out)
         return SOMHIP_ERR_STATE;
     }
     somhip_model *M = A->model;
-    M->prepared = false;
+    M->weights_changed();
     return somhip_launch_divide(M->ctx->stream, A->acc, M->mn, M->dim, model_w<T>(M), history_out);
 }
 
@@ -566,39 +588,21 @@ int somhip_model_create(somhip_ctx *C, int m, int n, int dim, int topology, cons
     M->topology = topology;
     M->nblk = (M->mn + 31) / 32;
     M->separable = closed_form_grid(topo_host, m, n, topology);
-    PermLayout layout = make_perm(m, n);
-    M->pblk = layout.pblk;
-    M->pblk_a = layout.pblk_a;
     const size_t slots = (size_t)M->nblk * 32;
-    const size_t pslots = (size_t)M->pblk * 32;
-    auto fail = [&](hipError_t e, const char *what) {
-        somhip_set_error(std::string(what) + ": " + hipGetErrorString(e));
+    hipError_t e;
+    if ((e = hipMalloc((void **)&M->w, sizeof(float) * M->mn * dim)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->topo, sizeof(float) * M->mn * 2)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->norms_nat, sizeof(float) * slots)) != hipSuccess ||
+        (e = hipMalloc((void **)&M->frag_f32, sizeof(float) * slots * M->dpad)) != hipSuccess ||
+        (e = alloc_search(M, sizeof(float))) != hipSuccess ||
+        (e = hipMemcpyAsync(M->topo, topo_host, sizeof(float) * M->mn * 2, hipMemcpyHostToDevice, C->stream)) !=
+            hipSuccess ||
+        (e = hipMemsetAsync(M->w, 0, sizeof(float) * M->mn * dim, C->stream)) != hipSuccess ||
+        (e = hipStreamSynchronize(C->stream)) != hipSuccess) {
+        somhip_set_error(std::string("float32 model: ") + hipGetErrorString(e));
         somhip_model_destroy(M);
         return SOMHIP_ERR_HIP;
-    };
-    hipError_t e;
-#define SOM_ALLOC(ptr, bytes)                                  \
-    if ((e = hipMalloc((void **)&(ptr), (bytes))) != hipSuccess) \
-        return fail(e, "hipMalloc");
-    SOM_ALLOC(M->w, sizeof(float) * M->mn * dim);
-    SOM_ALLOC(M->topo, sizeof(float) * M->mn * 2);
-    SOM_ALLOC(M->centre, sizeof(float) * M->dpad);
-    SOM_ALLOC(M->wmax, sizeof(float) * M->dpad);
-    SOM_ALLOC(M->scal, sizeof(float) * 4);
-    SOM_ALLOC(M->norms_perm, sizeof(float) * pslots);
-    SOM_ALLOC(M->norms_nat, sizeof(float) * slots);
-    SOM_ALLOC(M->frag_bf, sizeof(unsigned short) * pslots * M->dpad * 2);
-    SOM_ALLOC(M->frag_f32, sizeof(float) * slots * M->dpad);
-    SOM_ALLOC(M->wslot, sizeof(float) * pslots * M->dpad);
-    SOM_ALLOC(M->perm, sizeof(int) * pslots);
-#undef SOM_ALLOC
-    if ((e = hipMemcpyAsync(M->perm, layout.perm.data(), sizeof(int) * pslots, hipMemcpyHostToDevice, C->stream)) != hipSuccess)
-        return fail(e, "hipMemcpy perm");
-    if ((e = hipMemcpyAsync(M->topo, topo_host, sizeof(float) * M->mn * 2, hipMemcpyHostToDevice, C->stream)) != hipSuccess)
-        return fail(e, "hipMemcpy topography");
-    if ((e = hipMemsetAsync(M->w, 0, sizeof(float) * M->mn * dim, C->stream)) != hipSuccess) return fail(e, "hipMemset");
-    if ((e = hipStreamSynchronize(C->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
-    M->prepared = false;
+    }
     *out = M;
     return SOMHIP_OK;
 }
@@ -607,8 +611,8 @@ int somhip_model_destroy(somhip_model *M)
 {
     if (!M) return SOMHIP_OK;
     if (M->ctx) (void)hipStreamSynchronize(M->ctx->stream);
-    void *ptrs[] = {M->w,         M->topo,    M->centre,   M->wmax,  M->scal, M->norms_perm,
-                    M->norms_nat, M->frag_bf, M->frag_f32, M->wslot, M->perm, M->w64, M->topo64};
+    void *ptrs[] = {M->w,     M->topo,  M->centre, M->basis,    M->rot,  M->plan, M->wrot,  M->norms,
+                    M->frag_h, M->wslot, M->perm,  M->norms_nat, M->frag_f32, M->w64, M->topo64};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete M;
@@ -626,7 +630,7 @@ int somhip_model_set_weights(somhip_model *M, const float *w, int on_device)
     SOM_HIP_TRY(hipMemcpyAsync(M->w, w, sizeof(float) * M->mn * M->dim,
                                on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, M->ctx->stream));
     if (!on_device) SOM_HIP_TRY(hipStreamSynchronize(M->ctx->stream));
-    M->prepared = false;
+    M->weights_changed();
     M->uploads++;  // earlier BMUs kept by accumulators no longer describe this map's schedule
     return SOMHIP_OK;
 }
@@ -764,7 +768,7 @@ int somhip_batch_epoch_accumulate(somhip_accum *A, const float *x, const double 
     Workspace &W = A->ws;
     precision = somhip_bmu_precision(M, precision);  // the per-wave |x| rows depend on the kernel that runs
     const int64_t xrows = somhip_bmu_xmax_rows(precision, M->dpad, n);
-    // the previous call's BMUs of the same samples (the previous epoch) guide the BF16 search's grouping
+    // the previous call's BMUs of the same samples (the previous epoch) guide the 16-bit search's grouping
     // (not after an explicit weight upload: a new schedule starts without them, as a new train() does)
     const bool have_prev = precision == SOMHIP_PREC_BF16_RERANK && W.c1_x == (const void *)x && W.c1_n == n &&
                            W.c1_uploads == M->uploads;
@@ -836,7 +840,7 @@ int somhip_batch_iter_update(somhip_accum *A, float *history_out)
 
 // ------------------------------------------------------------------------------------------------
 // float64 SOMs (the reference's dtype=np.float64): data, weights and topography in FP64; the BMU
-// search is the exact FP64 scan, the sums are the same fixed-point scatter, the update writes FP64.
+// search ends in the exact FP64 distance, the sums are the same fixed-point scatter, the update writes FP64.
 // ------------------------------------------------------------------------------------------------
 int somhip_model_create_f64(somhip_ctx *C, int m, int n, int dim, int topology, const double *topo_host,
                             somhip_model **out)
@@ -854,6 +858,7 @@ int somhip_model_create_f64(somhip_ctx *C, int m, int n, int dim, int topology, 
     hipError_t e;
     if ((e = hipMalloc((void **)&M->w64, sizeof(double) * M->mn * dim)) != hipSuccess ||
         (e = hipMalloc((void **)&M->topo64, sizeof(double) * M->mn * 2)) != hipSuccess ||
+        (e = alloc_search(M, sizeof(double))) != hipSuccess ||
         (e = hipMemcpyAsync(M->topo64, topo_host, sizeof(double) * M->mn * 2, hipMemcpyHostToDevice, C->stream)) !=
             hipSuccess ||
         (e = hipMemsetAsync(M->w64, 0, sizeof(double) * M->mn * dim, C->stream)) != hipSuccess ||
@@ -877,6 +882,7 @@ int somhip_model_set_weights_f64(somhip_model *M, const double *w, int on_device
     SOM_HIP_TRY(hipMemcpyAsync(M->w64, w, sizeof(double) * M->mn * M->dim,
                                on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, M->ctx->stream));
     if (!on_device) SOM_HIP_TRY(hipStreamSynchronize(M->ctx->stream));
+    M->weights_changed();
     M->uploads++;
     return SOMHIP_OK;
 }

@@ -13,7 +13,7 @@
 // ------------------------------------------------------------------------------------------------
 // Vector types for the MFMA builtins.
 // ------------------------------------------------------------------------------------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
@@ -21,23 +21,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 #define SOM_FLOAT_EPS 1.0e-12
 
-// 32x32 MFMA accumulator layout (v_mfma_f32_32x32x{2f32,16_bf16}): lane l, register r holds
+// 32x32 MFMA accumulator layout (v_mfma_f32_32x32x{2f32,16_f16}): lane l, register r holds
 // D[row][col] with col = l % 32 and row = 8*(r/4) + 4*(l/32) + (r%4).
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
-
-// Round-to-nearest-even float -> bf16 bits (NaN kept quiet).
-__host__ __device__ __forceinline__ unsigned short f32_to_bf16_bits(float f)
-{
-    unsigned int u = __builtin_bit_cast(unsigned int, f);
-    if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x007FFFFFu)) return (unsigned short)((u >> 16) | 0x40u);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
-
-__host__ __device__ __forceinline__ float bf16_bits_to_f32(unsigned short b)
-{
-    return __builtin_bit_cast(float, (unsigned int)b << 16);
-}
 
 // The reference's square_distance_xpu (decontamination/algo/__init__.py:89-98): FP32 difference,
 // FP32 square (numba types float32 ** int as float32), FP64 sequential accumulation.
@@ -112,16 +98,32 @@ struct Top2 {
 // ------------------------------------------------------------------------------------------------
 // Descriptors shared by the BMU kernels and the serving loop.
 // ------------------------------------------------------------------------------------------------
-// Everything the BF16 kernel needs to know about one prepared model.
+// What the 16-bit search knows about one prepared map, on the device: the split plan and the maxima its
+// error bound is made of (float bits raised by atomicMax). Squares of lengths, in units of 2^-2k.
+constexpr int F16_MAX_DIM = 64;
+struct BmuPlan {
+    unsigned int wmax[F16_MAX_DIM];  // max_j |w''_ji| per direction (unscaled), index half * kpad/2 + t
+    unsigned int nw2;                // max_j |w'_j|^2
+    unsigned int lt2, nt2, rt2;      // split directions: max_j |low part|^2, |w''|^2, |remainder|^2
+    unsigned int ns2, rs2;           // directions held by their high part alone: |w''|^2, |remainder|^2
+    unsigned int nd2;                // directions left out: |w''|^2
+    unsigned int rn;                 // max_j remainder of the split norm
+    float defect;                    // Frobenius norm of (rotation^T rotation - 1)
+    float s1;                        // sum over the directions of max_j |w''_ji| (unscaled; rotated plans)
+    int rotated;                     // directions are those of the rotation (else the data's own dimensions)
+    int nk;                          // K slices of 16 per block
+    int q3h;                         // split directions per lane half
+    int k;                           // weights are scaled by 2^k
+};
+
+// Everything the 16-bit search kernel needs to know about one prepared model.
 struct BmuModelDev {
-    const bf16x8 *frag;     // bf16 A fragments (permuted slots)
-    const f32x4 *norms4;    // |w'|^2 per permuted slot
+    const f16x8 *frag;      // FP16 A fragments (permuted slots)
+    const float *rot;       // rotation as FP32 MFMA A operands [dpad/16][64 lanes][8]
+    const BmuPlan *plan;
     const int *perm;        // slot -> neuron
-    const float *w;         // FP32 weights (mn, dim)
-    const float *centre;    // weight centroid (dpad)
-    const float *wmax;      // max_j |w'_jk| (dpad)
-    const float *scal;      // [0] max_j |w'_j|^2
-    const float *wslot;     // FP32 weights (as given) per permuted slot, (slots, dpad), zero padded
+    const float *centre;    // weight centroid (kpad)
+    const void *wslot;      // weights (as given, float or double) per permuted slot, (slots, kpad), zero padded
     int nblk;               // 32-slot blocks of the permuted order
     int nblk_a;             // leading blocks that hold the coarse sub-lattice (== nblk: none)
     int mn, dim;
@@ -140,7 +142,7 @@ struct BmuTile {
     int default_index;
 };
 
-constexpr int SOM_TILE_ROWS = 512;     // rows per BF16 workgroup (8 waves x 2 groups x 32)
+constexpr int SOM_TILE_ROWS = 512;     // rows per search workgroup (8 waves x 2 groups x 32)
 constexpr int FB_TILE_SHIFT = 40;      // serving fallback entry = (tile << 40) | row
 
 // ------------------------------------------------------------------------------------------------
@@ -183,7 +185,7 @@ struct DevBuf {
 struct Workspace {
     DevBuf c1, c2, d1, part, bounds, shifts, table, xmax, maps, bucket;
     // Training: c1b holds the BMUs of the previous epoch_accumulate call, whose samples were c1_x / c1_n;
-    // the BF16 search groups each tile's rows by them (a stale buffer only changes the grouping's speed).
+    // the 16-bit search groups each tile's rows by them (a stale buffer only changes the grouping's speed).
     DevBuf c1b;
     const void *c1_x = nullptr;
     int64_t c1_n = -1;
@@ -233,29 +235,34 @@ struct somhip_ctx {
 struct somhip_model {
     somhip_ctx *ctx = nullptr;
     int m = 0, n = 0, mn = 0, dim = 0, dpad = 0, topology = SOMHIP_TOPOLOGY_HEXAGONAL;
+    int kpad = 0;           // padded dimension of the search's rows: 16, 32 or 64
     bool separable = false; // topography is the closed-form square / hexagonal grid (separable neighbourhood)
-    int nblk = 0;          // number of 32-neuron blocks in natural order (mn rounded up to 32)
-    int pblk = 0;          // number of 32-slot blocks in the permuted (BF16) order
-    int pblk_a = 0;        // leading permuted blocks holding the coarse sub-lattice (== pblk: none)
-    float *w = nullptr;    // (mn, dim) FP32 weights, row-major
-    float *topo = nullptr; // (mn, 2) FP32 topography
-    // float64 models (somhip_model_create_f64) hold their weights and topography here instead and have
-    // none of the FP32 buffers or prepared data
+    int nblk = 0;           // number of 32-neuron blocks in natural order (mn rounded up to 32)
+    int pblk = 0;           // number of 32-slot blocks in the permuted order
+    int pblk_a = 0;         // leading permuted blocks holding the coarse sub-lattice (== pblk: none)
+    float *w = nullptr;     // (mn, dim) FP32 weights, row-major
+    float *topo = nullptr;  // (mn, 2) FP32 topography
+    // float64 models (somhip_model_create_f64) hold their weights and topography here instead
     bool f64 = false;
     double *w64 = nullptr;
     double *topo64 = nullptr;
-    long long uploads = 0; // weight uploads by the caller (set_weights); an epoch's own update does not count
-    // prepared data (valid when prepared == true)
-    bool prepared = false;
-    float *centre = nullptr;        // (dpad) FP32 centroid of the weights
-    float *wmax = nullptr;          // (dpad) max_j |w'_jk|
-    float *scal = nullptr;          // [0] = max_j |w'_j|^2 (as float)
-    float *norms_perm = nullptr;    // (pblk*32) |w'|^2 in permuted slot order (padding slots = +inf)
-    float *norms_nat = nullptr;     // (nblk*32) |w'|^2 in natural order (padding slots = +inf)
-    unsigned short *frag_bf = nullptr;  // bf16 A fragments [blk][kc][hi,lo][64 lanes][8]
-    float *frag_f32 = nullptr;      // FP32 A fragments [blk][dpad/8][64 lanes][4]
-    float *wslot = nullptr;         // FP32 weights (as given) per permuted slot [slot][dpad], zero padded
+    long long uploads = 0;  // weight uploads by the caller (set_weights); an epoch's own update does not count
+    // prepared data of the 16-bit search: 0 none, 1 in the data's own dimensions, 2 rotated
+    int prepared = 0;
+    float *centre = nullptr;        // (kpad) FP32 centroid of the weights
+    double *basis = nullptr;        // (kpad, kpad) rotation, one direction per row
+    float *rot = nullptr;           // the same as FP32 MFMA A operands
+    BmuPlan *plan = nullptr;
+    float *wrot = nullptr;          // (pblk*32, kpad) rotated centred weights per permuted slot
+    double *norms = nullptr;        // (pblk*32) |w'|^2
+    _Float16 *frag_h = nullptr;     // FP16 A fragments [blk][nk][64 lanes][8]
+    void *wslot = nullptr;          // weights (as given) per permuted slot [slot][kpad], zero padded
     int *perm = nullptr;            // (pblk*32) slot -> neuron (or -1 for padding)
+    // prepared data of the plain FP32 search (float32 models; valid when prepared_f32 == true)
+    bool prepared_f32 = false;
+    float *norms_nat = nullptr;     // (nblk*32) |w'|^2 in natural order (padding slots = +inf)
+    float *frag_f32 = nullptr;      // FP32 A fragments [blk][dpad/8][64 lanes][4]
+    void weights_changed() { prepared = 0; prepared_f32 = false; }
 };
 
 // Timing helpers: bracket a launch with timer_begin / timer_end (no-ops unless enabled).
@@ -269,26 +276,35 @@ struct TimerScope {
 int somhip_timer_collect(somhip_ctx *C);
 
 // Internal launchers (return SOMHIP_OK or an error code).
-int somhip_prepare(somhip_model *mdl);
+// for the 16-bit search over about `n` rows (a longer search is worth a rotated basis)
+int somhip_prepare(somhip_model *mdl, int64_t n);
+int somhip_prepare_f32(somhip_model *mdl);  // for the plain FP32 search
 // The BMU precision a launch with `precision` runs on this model (BF16_RERANK maps beyond 65,504
 // neuron slots run the exact kernel, which returns the same winners).
 int somhip_bmu_precision(const somhip_model *mdl, int precision);
 // xmax_part (nullable): per-wave rows of dpad floats with max |x_k| over finite values, for the
 // fixed-point scales of training; somhip_bmu_xmax_rows gives the number of rows written.
-// fb_list / fb_count (nullable, both or neither): the BF16 path's fallback workspace (n int64 entries and
+// fb_list / fb_count (nullable, both or neither): the 16-bit search's fallback workspace (n int64 entries and
 // one counter); when absent the context's grow-only workspace is used (and allocated if too small).
-// prev_c1 (nullable, must not alias c1): earlier BMUs of the same rows; the BF16 search groups each
+// prev_c1 (nullable, must not alias c1): earlier BMUs of the same rows; the 16-bit search groups each
 // tile's rows by them, which changes only its speed, never its results.
 int somhip_launch_bmu(somhip_model *mdl, const float *x, int64_t n, int precision, int arithmetic, int need_c2,
                       int default_index, int32_t *c1, int32_t *c2, double *d1, float *xmax_part,
                       int64_t *fb_list = nullptr, unsigned int *fb_count = nullptr,
                       const int32_t *prev_c1 = nullptr);
 int64_t somhip_bmu_xmax_rows(int precision, int dpad, int64_t n);
-// Exact FP64 search of a float64 model (data and weights in FP64); same output contract.
+// The search of a float64 model (data and weights in FP64, exact FP64 rerank); same output contract.
 int somhip_launch_bmu_f64(somhip_model *mdl, const double *x, int64_t n, int need_c2, int default_index, int32_t *c1,
                           int32_t *c2, double *d1);
+constexpr int f16_max_nk(int kpad) { return kpad <= 16 ? 2 : kpad <= 32 ? 3 : 5; }
+// Most K slices a plan of this model may take: rotated directions spread evenly over the lane halves, so up to 46 of
+// them fit three slices (23 slots a half); the data's own dimensions do not.
+inline int f16_nk_limit(const somhip_model *M, bool rotated)
+{
+    return M->kpad == 64 && rotated && M->dim <= 46 ? 3 : f16_max_nk(M->kpad);
+}
 BmuModelDev somhip_model_dev(const somhip_model *M);
-// Serving form of the BF16 search: `grid` tiles from `tiles` (n == 0 tiles are skipped), then the exact
+// Serving form of the 16-bit search: `grid` tiles from `tiles` (n == 0 tiles are skipped), then the exact
 // fallback over the flagged (tile, row) entries with a fixed grid; fb_count must be zero on entry.
 int somhip_launch_bmu_tiles(hipStream_t st, int dpad, int arithmetic, int need_c2, const BmuModelDev *models,
                             const BmuTile *tiles, int grid, int64_t *fb_list, unsigned int *fb_count);

@@ -126,8 +126,19 @@ __global__ __launch_bounds__(1024) void shifts_parts_kernel(const float *__restr
     const int r0 = threadIdx.x / dpad;
     const int rs = blockDim.x / dpad;
     float m = 0.f;
-    if (r0 < rs)
-        for (int64_t r = r0; r < rows; r += rs) m = fmaxf(m, parts[r * dpad + k]);
+    if (r0 < rs) {
+        // 16 loads in flight: one block, so the loop is a chain of load latencies
+        int64_t r = r0;
+        for (; r + 15 * (int64_t)rs < rows; r += 16 * (int64_t)rs) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) v[u] = parts[(r + u * (int64_t)rs) * dpad + k];
+#pragma unroll
+            for (int u = 0; u < 16; u++) m = fmaxf(m, v[u]);
+        }
+#pragma unroll 4
+        for (; r < rows; r += rs) m = fmaxf(m, parts[r * dpad + k]);
+    }
     red[threadIdx.x] = m;
     __syncthreads();
     if ((int)threadIdx.x <= dim) {
@@ -785,8 +796,9 @@ int somhip_launch_shifts(hipStream_t st, const unsigned long long *bounds, int d
 int somhip_launch_shifts_parts(hipStream_t st, const float *parts, int64_t rows, int dpad, int dim,
                                const unsigned long long *rho_bound, int64_t n, int *shifts)
 {
-    // first stage: fold the rows in place into the first RB rows (RB x dpad maxima), then one block
-    constexpr int RB = 2048;
+    // first stage: fold the rows in place into the first RB rows (RB x dpad maxima), then one block. 4096 rows of
+    // 16 values are four chains of 16 loads per thread, about what the extra launch costs.
+    constexpr int RB = 4096;
     if (rows > RB) {
         hipLaunchKernelGGL(rowmax_fold_kernel, dim3(RB), dim3(256), 0, st, (float *)parts, rows, dpad, RB);
         SOM_HIP_TRY(hipGetLastError());

@@ -603,7 +603,7 @@ int somhip_server_add_model(somhip_server *S, somhip_model *M, int *model_id)
         somhip_set_error("serving supports at most 65504 neuron slots (about 65,000 neurons)");
         return SOMHIP_ERR_UNSUPPORTED;
     }
-    int rc = somhip_prepare(M);
+    int rc = somhip_prepare(M, INT64_MAX / M->mn);  // resident: always worth the rotated basis
     if (rc) return rc;
     SOM_HIP_TRY(hipStreamSynchronize(M->ctx->stream));
     BmuModelDev d = somhip_model_dev(M);

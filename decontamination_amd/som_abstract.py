@@ -6,14 +6,14 @@ Mirrors ``decontamination.algo.som_abstract.SOM_Abstract``
 ``compute_errors``, ``get_activation_map`` and ``get_winners`` with the same arguments, return
 types and dtypes. Additive keyword-only options select the BMU search precision:
 
-  precision  'bf16_rerank' (default) split-BF16 MFMA distance GEMM + exact rerank: the BMUs equal the
+  precision  'bf16_rerank' (default) split 16-bit MFMA distance GEMM + exact rerank: the BMUs equal the
              reference formula's on every sample; 'fp32' plain FP32 MFMA GEMM; 'exact' direct scan.
   arithmetic 'ref32' (default) the reference's distance arithmetic (FP32 difference and square, FP64
              sum); 'fp64' FP64 throughout.
 
 ``dtype=np.float64`` keeps weights, topography, data and sums in FP64 on the device, as the
-reference's float64 SOMs do; their search is the exact FP64 scan (precision 'exact', arithmetic
-'fp64', the only values such a SOM takes). float32 and float64 are the dtypes the GPU path supports.
+reference's float64 SOMs do; their search returns the exact FP64 distance's winners (precision
+'exact', arithmetic 'fp64', the only values such a SOM takes). float32 and float64 are the dtypes the GPU path supports.
 
 This package is the GPU path only. ``enable_gpu=False`` raises: the CPU path stays the reference's
 own. ``threads_per_blocks`` is accepted for signature compatibility and ignored (launch shapes are

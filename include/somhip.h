@@ -42,7 +42,7 @@ extern "C" {
 /* BMU search precision. */
 #define SOMHIP_PREC_EXACT 0       /* direct-difference scan on the vector ALUs, rerank arithmetic below */
 #define SOMHIP_PREC_FP32 1        /* plain FP32 MFMA distance GEMM |w|^2 - 2 x.w, argmin on its values */
-#define SOMHIP_PREC_BF16_RERANK 2 /* 3-term split-BF16 MFMA GEMM, provable candidate window, exact rerank;
+#define SOMHIP_PREC_BF16_RERANK 2 /* split 16-bit MFMA GEMM, provable candidate window, exact rerank;
                                     maps beyond 65,504 neuron slots run PREC_EXACT (same winners) */
 
 /* Arithmetic of the exact distance (PREC_EXACT and the rerank of PREC_BF16_RERANK). */
@@ -133,12 +133,12 @@ int somhip_find_bmus(somhip_model *model, const float *x, int64_t n, int precisi
 
 /* Winners, as somhip_find_bmus, without allocating: no hipMalloc/hipFree or other allocation inside the
  * call (kernel timers are suspended for its duration). No counterpart in the reference: it is for callers
- * that cannot allocate, such as code under HIP graph capture and serving loops. The BF16 path's fallback
+ * that cannot allocate, such as code under HIP graph capture and serving loops. The 16-bit search's fallback
  * list lives in a fixed device array of 256 + 8 * SOMHIP_NOALLOC_MAX_ROWS bytes (16 MB) that every device
  * holds for the life of the process, cleared by a kernel at the start of each call; n above
  * SOMHIP_NOALLOC_MAX_ROWS is rejected with SOMHIP_ERR_ARG (split the input). All calls on one device share
  * that array: calls that overlap on one device (several contexts or streams at once) race. When the weights
- * changed since the last search, the call first rebuilds the model's derived data with the prep kernels,
+ * changed since the last search, or this is the first one long enough to rotate them, the call first rebuilds the model's derived data with the prep kernels,
  * in the model's own buffers. */
 #define SOMHIP_NOALLOC_MAX_ROWS (1 << 21)
 int somhip_find_bmus_noalloc(somhip_model *model, const float *x, int64_t n, int precision, int arithmetic,
@@ -217,7 +217,7 @@ int somhip_batch_iter_update(somhip_accum *acc, float *history_out);
  * float64 SOMs: the reference's dtype=np.float64 (som_abstract.py:46-68, som_batch.py:289-291,
  * 311-315), where weights, topography, data (`vectors.astype(dtype)`), sigma and the sums are FP64.
  * A float64 model holds FP64 weights and topography; its entry points take FP64 device rows and
- * search with the exact FP64 scan (the reference's square_distance_xpu on float64 operands:
+ * search by the exact FP64 distance (the reference's square_distance_xpu on float64 operands:
  * FP64 difference, square and sequential sum), so they have no precision/arithmetic arguments.
  * The per-BMU sums are the same exact fixed-point sums of the FP64 products rho*x; the density is not
  * rounded. The update computes the neighbourhood from FP64 topography differences and writes FP64
