@@ -146,10 +146,14 @@ __device__ __forceinline__ void wave_dim_max(const float (&amax)[8], int kc, boo
 // ------------------------------------------------------------------------------------------------
 constexpr int NW_F16 = 8;       // waves per workgroup
 constexpr int G_F16 = 2;        // 32-sample groups per wave
-// Short searches take tiles of 4 waves with one group each: at 512 rows a tile, 131,072 rows make one workgroup
-// per CU and fewer leave CUs idle. Longer ones keep the large tile, whose fragment traffic per row is a quarter.
+// Short searches take tiles of one group per wave: at 512 rows a tile, 131,072 rows make one workgroup per CU and
+// fewer leave CUs idle. 4 waves a tile as long as all tiles fit the 256 CUs at once (three a CU), then 8 waves:
+// errors of 98,000 rows on 64x64 at D = 16 take 119 us in tiles of 4 waves and 145 us in large ones; of 131,000 rows 173
+// us in tiles of 4 waves, 130 us in tiles of 8 and 148 us in large ones. Longer ones keep the large tile, whose
+// fragment traffic per row is a half: 500,000 rows take 319 us, 352 us in tiles of 8 waves and one group.
 constexpr int NW_SMALL = 4;
-constexpr int64_t SMALL_ROWS = 131072;
+constexpr int64_t SMALL_ROWS = 3 * 256 * NW_SMALL * 32;
+constexpr int64_t MEDIUM_ROWS = 131072;
 constexpr int FRAG_UNITS = 1024; // 16-byte units of A fragments per chunk buffer
 static_assert(NW_F16 * G_F16 * 32 == SOM_TILE_ROWS, "tile rows must match the search workgroup");
 
@@ -213,11 +217,9 @@ template <int HD>
 using HalfDirs = float __attribute__((ext_vector_type(HD)));
 
 // One half wave's B slots from its scaled directions: the first Q3 as (high, low, high), then high parts; sums the
-// squares of what the products leave out: low parts (lt) and remainders (rt) of the split directions,
-// remainders (rs) of the others.
+// squares of the remainders of the latter (rs).
 template <int NK, int HD, int Q3>
-__device__ __forceinline__ void build_slots(HalfDirs<HD> xi, float norm_mult, f16x8 (&b)[NK], float &lt,
-                                            float &rt, float &rs)
+__device__ __forceinline__ void build_slots(HalfDirs<HD> xi, float norm_mult, f16x8 (&b)[NK], float &rs)
 {
     constexpr int Q1 = F16Split<NK, HD>::q1(Q3);
 #pragma unroll
@@ -227,11 +229,7 @@ __device__ __forceinline__ void build_slots(HalfDirs<HD> xi, float norm_mult, f1
 #pragma unroll
     for (int t = 0; t < Q3; t++) {
         const _Float16 h = (_Float16)xi[t];
-        const float r1 = xi[t] - (float)h;
-        const _Float16 l = (_Float16)r1;
-        const float lf = (float)l, r2 = r1 - lf;
-        lt = fmaf(lf, lf, lt);
-        rt = fmaf(r2, r2, rt);
+        const _Float16 l = (_Float16)(xi[t] - (float)h);
         b[(3 * t) / 8][(3 * t) % 8] = h;
         b[(3 * t + 1) / 8][(3 * t + 1) % 8] = l;
         b[(3 * t + 2) / 8][(3 * t + 2) % 8] = h;
@@ -249,13 +247,12 @@ __device__ __forceinline__ void build_slots(HalfDirs<HD> xi, float norm_mult, f1
 }
 // The same for a plan's q3 (uniform).
 template <int NK, int HD, int Q3 = F16Split<NK, HD>::QMIN>
-__device__ __forceinline__ void build_slots_q(int q3, HalfDirs<HD> xi, float norm_mult, f16x8 (&b)[NK], float &lt,
-                                              float &rt, float &rs)
+__device__ __forceinline__ void build_slots_q(int q3, HalfDirs<HD> xi, float norm_mult, f16x8 (&b)[NK], float &rs)
 {
     if constexpr (Q3 < F16Split<NK, HD>::QMAX) {
-        if (q3 != Q3) return build_slots_q<NK, HD, Q3 + 1>(q3, xi, norm_mult, b, lt, rt, rs);
+        if (q3 != Q3) return build_slots_q<NK, HD, Q3 + 1>(q3, xi, norm_mult, b, rs);
     }
-    build_slots<NK, HD, Q3>(xi, norm_mult, b, lt, rt, rs);
+    build_slots<NK, HD, Q3>(xi, norm_mult, b, rs);
 }
 
 // Power of two 2^e for |e| <= 126.
@@ -491,10 +488,8 @@ __device__ __forceinline__ void bmu_f16_body(const BmuModelDev &Md, const T *__r
             const float sc = exp2i(ex);
 #pragma unroll
             for (int t = 0; t < HD; t++) xi[t] *= sc;
-            float lt = 0.f, rt = 0.f, rs = 0.f;
-            build_slots_q<NK, HD>(q3h, xi, exp2i(max(nm, -14)), bx[g], lt, rt, rs);
-            lt = __builtin_amdgcn_sqrtf(sum32(lt));
-            rt = __builtin_amdgcn_sqrtf(sum32(rt));
+            float rs = 0.f;
+            build_slots_q<NK, HD>(q3h, xi, exp2i(max(nm, -14)), bx[g], rs);
             rs = __builtin_amdgcn_sqrtf(sum32(rs));
             // Error bound of a_j, in units of 2^-(kw + ex):
             //   products left out: 2 (|remainder of x| |w| + |x| |remainder of w| + |low x| |low w|) per class
@@ -505,7 +500,10 @@ __device__ __forceinline__ void bmu_f16_body(const BmuModelDev &Md, const T *__r
             //   rounding of the rotated weights 2 (16 nk + 5) 2^-24 (|w|^2 + 2|x||w|); remainder of the norm;
             //   centring 4*2^-24 (|x|^2 + |w|^2).
             // 10% on top for the roundings of this arithmetic itself.
+            //   Low parts of x are at most 2^-11 of it and its remainders 2^-22, but for 2^-25 a direction where
+            //   they are subnormal; the remainders of directions without a low part are summed (rs).
             const float X = __builtin_amdgcn_sqrtf(kk) * (1.f + 4.f * U32) * sc;
+            const float lt = 4.9e-4f * X + 2.4e-7f, rt = 2.5e-7f * X + 2.4e-7f;
             const float back = exp2i(min(max(ex - kw, -126), 126));
             const float ns = nw_s * nw_s * back;
             const float kks = X * X * exp2i(min(max(kw - ex, -126), 126));
@@ -865,15 +863,13 @@ __device__ __forceinline__ void bmu_f16_run(const BmuModelDev &Md, const T *x, i
     if constexpr (NKMAX >= 5) {
         if (nk == 5) return run(integral_constant<int, 5>{});
     }
-    if constexpr (NKMAX >= 3) {
-        if (nk == 3) return run(integral_constant<int, 3>{});
-    }
+    if (nk == 3) return run(integral_constant<int, 3>{});
     run(integral_constant<int, 2>{});
 }
 
-// 4 waves per SIMD (3 of the small tiles, by their LDS)
+// 4 waves per SIMD (3 of the small tiles, by their LDS; 6 of those of 8 waves and one group at D = 16)
 template <int DP, int NKMAX, int NW, int G, int MODE, bool NEED_C2, class T>
-__global__ __launch_bounds__(NW * WAVE, NW == NW_F16 ? 4 : 3) void bmu_f16_kernel(BmuModelDev Md, const T *__restrict__ x, int64_t n,
+__global__ __launch_bounds__(NW * WAVE, NW == NW_SMALL ? 3 : G == 1 && DP == 16 ? 6 : 4) void bmu_f16_kernel(BmuModelDev Md, const T *__restrict__ x, int64_t n,
                                                                    int default_index, int32_t *__restrict__ c1,
                                                                    int32_t *__restrict__ c2, double *__restrict__ d1,
                                                                    int64_t *__restrict__ fb_list,
@@ -1027,6 +1023,8 @@ int somhip_search_f16(somhip_model *M, const T *x, int64_t n, int arithmetic, in
         const bool three = NKMAX > 3 && f16_nk_limit(M, M->prepared == 2) == 3;
         if (n <= SMALL_ROWS) {
             launch(integral_constant<int, NKMAX>{}, integral_constant<int, NW_SMALL>{}, integral_constant<int, 1>{});
+        } else if (n <= MEDIUM_ROWS) {
+            launch(integral_constant<int, NKMAX>{}, integral_constant<int, NW_F16>{}, integral_constant<int, 1>{});
         } else if (three) {
             if constexpr (NKMAX > 3)
                 launch(integral_constant<int, 3>{}, integral_constant<int, NW_F16>{}, integral_constant<int, G_F16>{});

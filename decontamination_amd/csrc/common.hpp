@@ -103,6 +103,7 @@ struct Top2 {
 constexpr int F16_MAX_DIM = 64;
 struct BmuPlan {
     unsigned int wmax[F16_MAX_DIM];  // max_j |w''_ji| per direction (unscaled), index half * kpad/2 + t
+    float step2[F16_MAX_DIM];        // sum over neighbours (j, j + 1) of one map row of (w_jk - w_j+1,k)^2, per data dimension
     unsigned int nw2;                // max_j |w'_j|^2
     unsigned int lt2, nt2, rt2;      // split directions: max_j |low part|^2, |w''|^2, |remainder|^2
     unsigned int ns2, rs2;           // directions held by their high part alone: |w''|^2, |remainder|^2
@@ -296,7 +297,7 @@ int64_t somhip_bmu_xmax_rows(int precision, int dpad, int64_t n);
 // The search of a float64 model (data and weights in FP64, exact FP64 rerank); same output contract.
 int somhip_launch_bmu_f64(somhip_model *mdl, const double *x, int64_t n, int need_c2, int default_index, int32_t *c1,
                           int32_t *c2, double *d1);
-constexpr int f16_max_nk(int kpad) { return kpad <= 16 ? 2 : kpad <= 32 ? 3 : 5; }
+constexpr int f16_max_nk(int kpad) { return kpad <= 32 ? 3 : 5; }
 // Most K slices a plan of this model may take: rotated directions spread evenly over the lane halves, so up to 46 of
 // them fit three slices (23 slots a half); the data's own dimensions do not.
 inline int f16_nk_limit(const somhip_model *M, bool rotated)

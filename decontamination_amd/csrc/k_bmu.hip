@@ -260,18 +260,24 @@ __global__ __launch_bounds__(BMU_WAVES * WAVE) void bmu_fp32_kernel(
 // fragments and the maxima of what they leave out.
 // ------------------------------------------------------------------------------------------------
 template <class T>
-__global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ w, int mn, int dim, int dpad,
+__global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ w, int mn, int ncol, int dim, int dpad,
                                                           float *__restrict__ centre, BmuPlan *__restrict__ plan)
 {
-    // one block per padded dimension; fixed-order FP64 sum, and the extent about the centroid. Also clears the
-    // maxima that the next kernels raise (same stream).
+    // one block per padded dimension; fixed-order FP64 sum, the extent about the centroid and the steps between
+    // neighbours of a map row (those within a wave). Also clears the maxima that the next kernels raise (same stream).
     const int k = blockIdx.x;
-    if (k == 0 && threadIdx.x >= F16_MAX_DIM && threadIdx.x < sizeof(BmuPlan) / sizeof(unsigned int))
+    if (k == 0 && threadIdx.x >= 2 * F16_MAX_DIM && threadIdx.x < sizeof(BmuPlan) / sizeof(unsigned int))
         ((unsigned int *)plan)[threadIdx.x] = 0u;
     __shared__ double red[256];
     __shared__ float mm[2][256];
     double acc = 0.0;
+    float st = 0.f;
     T lo = (T)__builtin_inf(), hi = -(T)__builtin_inf();
+    const bool last = (threadIdx.x & (WAVE - 1)) == WAVE - 1;
+    auto step = [&](int j, T v) {
+        const float d = (float)(__shfl_down(v, 1, WAVE) - v);
+        if (!last && j + 1 < mn && (j + 1) % ncol) st = fmaf(d, d, st);
+    };
     if (k < dim) {
         // 8 loads in flight, added in index order
         int j = threadIdx.x;
@@ -282,6 +288,7 @@ __global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ 
 #pragma unroll
             for (int u = 0; u < 8; u++) {
                 acc += (double)v[u];
+                step(j + u * 256, v[u]);
                 lo = fmin(lo, v[u]);
                 hi = fmax(hi, v[u]);
             }
@@ -289,6 +296,7 @@ __global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ 
         for (; j < mn; j += 256) {
             const T v = w[(int64_t)j * dim + k];
             acc += (double)v;
+            step(j, v);
             lo = fmin(lo, v);
             hi = fmax(hi, v);
         }
@@ -300,6 +308,9 @@ __global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ 
         __syncthreads();
     }
     const float c = (float)(red[0] / (double)mn);
+    __shared__ float steps[4];
+    for (int o = WAVE / 2; o > 0; o >>= 1) st += __shfl_xor(st, o, WAVE);
+    if (threadIdx.x % WAVE == 0) steps[threadIdx.x / WAVE] = st;
     // the centred extremes: subtraction and rounding are monotonic
     mm[0][threadIdx.x] = k < dim && lo <= hi ? fabsf(centred(lo, c)) : 0.f;
     mm[1][threadIdx.x] = k < dim && lo <= hi ? fabsf(centred(hi, c)) : 0.f;
@@ -310,6 +321,7 @@ __global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ 
         __syncthreads();
     }
     if (threadIdx.x == 0) {
+        plan->step2[k] = steps[0] + steps[1] + steps[2] + steps[3];
         centre[k] = k < dim ? c : 0.f;
         // dimension k is direction t = 8 (k / 16) + k % 8 of half (k / 8) % 2
         const int at = (k / 8 % 2) * (dpad / 2) + 8 * (k / 16) + k % 8;
@@ -320,20 +332,30 @@ __global__ __launch_bounds__(256) void prep_centre_kernel(const T *__restrict__ 
 // The rotation: an orthonormal basis of the row space, its leading directions close to the map's principal
 // ones. One workgroup: FP64 second moments C of up to basis_rows centred neurons (spread over the map by a
 // golden-ratio sequence, which no row or column of the map stays in step with), then a Householder
-// factorisation of C with column pivoting by the first wave, one column per lane in FP64, which applies every
-// reflection to the identity too. Any orthonormal basis gives correct bounds (the maxima are measured
-// afterwards, the departure from orthonormality here). On trained maps the bound comes within a quarter of the
-// eigenvectors'; FP32 moments lose the directions below 3e-4 of the first, which are left out and then cost
-// ten times the bound. Latency bound: a serial chain of up to dpad reflections.
-constexpr int BASIS_NT = 1024;
+// factorisation of C with column pivoting in FP64, which applies every reflection to the identity too. Any
+// orthonormal basis gives correct bounds (the maxima are measured afterwards, the departure from orthonormality
+// here). On trained maps the bound comes within a quarter of the eigenvectors'; with the neurons themselves as
+// pivots it is half as large again, and FP32 moments lose the directions below 3e-4 of the first.
+// Four lanes hold a column, a quarter of its values each. Latency bound: a serial chain of up to dpad steps of one
+// barrier each: 16, 31 and 84 us at
+// D = 16, 20 and 40 (one wave alone, a lane per column in LDS: 27, 60 and 182 us).
 template <int DP>
 constexpr int basis_rows() { return DP <= 32 ? 256 : 128; }
-template <int DP>
-constexpr size_t basis_lds()
+constexpr int BASIS_NT = 512;
+
+// Sum over the four lanes of a vector, in each of them.
+__device__ __forceinline__ double quad_sum(double v)
 {
-    const size_t mats = sizeof(double) * 2 * DP * (DP + 1);
-    const size_t rows = sizeof(float) * basis_rows<DP>() * (DP + 4) + sizeof(double) * 4 * BASIS_NT;
-    return mats > rows ? mats : rows;
+    auto dpp = [](double x, auto ctrl) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, x);
+        const int lo = (int)(unsigned)u, hi = (int)(unsigned)(u >> 32);
+        const unsigned a = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, decltype(ctrl)::value, 0xF, 0xF, true);
+        const unsigned b = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, decltype(ctrl)::value, 0xF, 0xF, true);
+        return __builtin_bit_cast(double, ((uint64_t)b << 32) | a);
+    };
+    v += dpp(v, std::integral_constant<int, 0xB1>{});  // quad_perm 1,0,3,2
+    v += dpp(v, std::integral_constant<int, 0x4E>{});  // quad_perm 2,3,0,1
+    return v;
 }
 
 template <int DP, class T>
@@ -346,105 +368,138 @@ __global__ __launch_bounds__(BASIS_NT) void prep_basis_kernel(const T *__restric
     constexpr int LD = DP + 1, LR = DP + 4;
     constexpr int QUADS = DP * DP / 4;          // (i, 4 k) groups of C
     constexpr int PARTS = BASIS_NT / QUADS > 0 ? BASIS_NT / QUADS : 1;  // row parts
-    static_assert(QUADS * PARTS == BASIS_NT, "one group of four per thread");
-    extern __shared__ double lds[];
-    double *A = lds;            // [DP][LD] C, reduced column by column
-    double *Q = A + DP * LD;    // [DP][LD] product of the reflections (rows: directions)
-    float *rows = (float *)lds; // [NR][LR] sampled rows, before A and Q
-    double *parts = (double *)(rows + NR * LR);  // [PARTS][QUADS][4]
-    __shared__ double vh[DP];
+    static_assert(QUADS * PARTS % BASIS_NT == 0, "whole groups of four per thread");
+    constexpr int R = DP / 4;             // values per lane
+    constexpr int NCW = 4 * DP / WAVE;    // waves of C's columns; the identity's follow
+    static_assert(2 * NCW * WAVE <= BASIS_NT, "a column per four threads");
+    // first the sampled rows, then the moments' parts, then the product of the reflections (rows: directions)
+    constexpr size_t ROWS_B = sizeof(float) * NR * LR, PARTS_B = sizeof(double) * PARTS * DP * DP, Q_B = sizeof(double) * DP * LD;
+    constexpr size_t LDS_B = ROWS_B > PARTS_B ? (ROWS_B > Q_B ? ROWS_B : Q_B) : (PARTS_B > Q_B ? PARTS_B : Q_B);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_B];
+    float *rows = (float *)lds;
+    double *parts = (double *)lds, *Q = (double *)lds;
+    __shared__ __attribute__((aligned(16))) double vb[2][NCW][DP];  // each wave's candidate
+    __shared__ float nb[2][NCW];                                    // and its squared length
     __shared__ float red[BASIS_NT / WAVE];
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE, vec = tid / 4, l = tid & 3;
+    // scaled to about one, so the moments and their squares stay in range
+    float big = lane < DP ? __builtin_bit_cast(float, plan->wmax[lane]) : 0.f;
+    for (int o = WAVE / 2; o > 0; o >>= 1) big = fmaxf(big, __shfl_xor(big, o, WAVE));
+    const float sc = big > 0.f && big < __builtin_inff() ? exp2i(min(126, max(-126, -expo(big)))) : 1.f;
     const int nr = min(mn, NR);
+#pragma unroll 8
     for (int e = tid; e < NR * DP; e += BASIS_NT) {
         const int r = e / DP, k = e % DP;
         const int j = mn <= NR ? min(r, mn - 1) : (int)(((uint64_t)((unsigned)r * 2654435769u) * (unsigned)mn) >> 32);
-        const float v = r < nr && k < dim ? centred(w[(int64_t)j * dim + k], centre[k]) : 0.f;
+        const float v = r < nr && k < dim ? centred(w[(int64_t)j * dim + k], centre[k]) * sc : 0.f;
         rows[r * LR + k] = __builtin_isfinite(v) ? v : 0.f;
     }
-    if (tid < F16_MAX_DIM) plan->wmax[tid] = 0u;  // the maxima of the rotated directions follow
     __syncthreads();
-    {
-        const int g = tid % QUADS, part = tid / QUADS, i = g / (DP / 4), k = 4 * (g % (DP / 4));
-        double c[4] = {0.0, 0.0, 0.0, 0.0};
+    if (tid < F16_MAX_DIM) plan->wmax[tid] = 0u;  // the maxima of the rotated directions follow
+    constexpr int PER = QUADS * PARTS / BASIS_NT;
+    double c[PER][4];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int at = tid + u * BASIS_NT, g = at % QUADS, part = at / QUADS, i = g / (DP / 4), k = 4 * (g % (DP / 4));
+#pragma unroll
+        for (int e = 0; e < 4; e++) c[u][e] = 0.0;
 #pragma unroll 8
         for (int r = part * (NR / PARTS); r < (part + 1) * (NR / PARTS); r++) {
             const double a = (double)rows[r * LR + i];
             const f32x4 b = *(const f32x4 *)&rows[r * LR + k];
 #pragma unroll
-            for (int e = 0; e < 4; e++) c[e] = fma(a, (double)b[e], c[e]);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) parts[4 * tid + e] = c[e];
-    }
-    __syncthreads();
-    constexpr int PER = DP * DP / BASIS_NT > 0 ? DP * DP / BASIS_NT : 1;
-    double cc[PER];
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-        const int e = tid + u * BASIS_NT;
-        cc[u] = 0.0;
-        if (e < DP * DP)
-            for (int q = 0; q < PARTS; q++) cc[u] += parts[q * DP * DP + e];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-        const int e = tid + u * BASIS_NT;
-        if (e < DP * DP) {
-            A[(e / DP) * LD + e % DP] = cc[u];
-            Q[(e / DP) * LD + e % DP] = e / DP == e % DP ? 1.0 : 0.0;
+            for (int e = 0; e < 4; e++) c[u][e] = fma(a, (double)b[e], c[u][e]);
         }
     }
     __syncthreads();
-    if (tid < WAVE) {
-        // lane: column of A and of Q; lanes past DP do nothing
-        const bool on = lane < DP;
-        bool used = !on;
-        const int steps = min(dim, DP - 1);
-        for (int i = 0; i < steps; i++) {
-            double best = used ? -1.0 : 0.0;
-            if (!used) {
-#pragma unroll 4
-                for (int r = i; r < DP; r++) best = fma(A[r * LD + lane], A[r * LD + lane], best);
-            }
-            int at = lane;
-            for (int o = (DP < WAVE ? DP : WAVE) / 2; o > 0; o >>= 1) {
-                const double pb = __shfl_xor(best, o, WAVE);
-                const int pa = __shfl_xor(at, o, WAVE);
-                if (pb > best || (pb == best && pa < at)) { best = pb; at = pa; }
-            }
-            best = __shfl(best, 0, WAVE);
-            at = __shfl(at, 0, WAVE);
-            if (!(best > 1e-280 && best < 1e280)) break;  // uniform: nothing left, the rest of the basis stays as it is
-            if (lane == at) used = true;
-            // v = column from row i on, its first value moved away from zero by its norm
-            const double head = A[i * LD + at];
-            const double len = sqrt(best);
-            const double v0 = head + (head >= 0.0 ? len : -len);
-            const double beta = 1.0 / (len * (len + fabs(head)));
-            if (lane >= i && lane < DP) vh[lane] = lane == i ? v0 : A[lane * LD + at];
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (on) {
-                double da = 0.0, dq = 0.0;
-#pragma unroll 4
-                for (int r = i; r < DP; r++) {
-                    da = fma(vh[r], A[r * LD + lane], da);
-                    dq = fma(vh[r], Q[r * LD + lane], dq);
-                }
-                da *= beta;
-                dq *= beta;
-#pragma unroll 4
-                for (int r = i; r < DP; r++) {
-                    A[r * LD + lane] = fma(-da, vh[r], A[r * LD + lane]);
-                    Q[r * LD + lane] = fma(-dq, vh[r], Q[r * LD + lane]);
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) parts[4 * (tid + u * BASIS_NT) + e] = c[u][e];
+    __syncthreads();
+    const bool isc = wave < NCW, on = wave < 2 * NCW;  // uniform over the wave
+    double x[R];
+    float nrm = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int k = l * R + r;
+        x[r] = 0.0;
+        if (isc) {
+            for (int q = 0; q < PARTS; q++) x[r] += parts[q * DP * DP + k * DP + vec];
+        } else if (on) {
+            x[r] = vec - DP == k ? 1.0 : 0.0;
         }
     }
+    auto length2 = [&]() {
+        double m = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; r++) m = fma(x[r], x[r], m);
+        nrm = (float)quad_sum(m);
+    };
+    length2();
+    __syncthreads();  // the moments have been read: Q takes their place
+    const int steps = min(dim, DP - 1);
+    float floor2 = 0.f;
+    int i = 0;
+    for (; i < steps; i++) {
+        const int buf = i & 1;
+        if (isc) {
+            float m = half_max(nrm), ma, mb;
+            pair32(m, ma, mb);
+            m = fmaxf(ma, mb);
+            const unsigned long long at_max = __builtin_amdgcn_ballot_w64(nrm == m);
+            const int top = at_max ? __builtin_ctzll(at_max) & ~3 : 0;
+            if ((lane & ~3) == top) {
+#pragma unroll
+                for (int r = 0; r < R; r++) vb[buf][wave][l * R + r] = x[r];
+                if (l == 0) nb[buf][wave] = m;
+            }
+        }
+        __syncthreads();  // two buffers: the next step's candidates are written while these are read
+        float best = nb[buf][0];
+        int s = 0;
+#pragma unroll
+        for (int q = 1; q < NCW; q++) {
+            const float m = nb[buf][q];
+            if (m > best) { best = m; s = q; }
+        }
+        // uniform: nothing left to the rounding of FP64, the rest of the basis stays as it is
+        if (!(best > floor2 && best < __builtin_inff())) break;
+        if (i == 0) floor2 = 1e-29f * best;
+        if (!on) continue;
+        s = __builtin_amdgcn_readfirstlane(s);
+        // v = the candidate (zero before value i), its value i moved away from zero by its length
+        const double head = vb[buf][s][i];
+        const int own = i - l * R;  // value i among this lane's
+        double v[R], d = 0.0, tail = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            v[r] = vb[buf][s][l * R + r];
+            if (r != own) tail = fma(v[r], v[r], tail);
+        }
+        tail = quad_sum(tail);
+        const double len = sqrt(fma(head, head, tail)), v0 = head + (head >= 0.0 ? len : -len);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (r == own) v[r] = v0;
+            d = fma(v[r], x[r], d);
+        }
+        const double f = -2.0 * quad_sum(d) / fma(v0, v0, tail);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            x[r] = fma(f, v[r], x[r]);
+            if (r == own) {
+                // final: a row of the product; of C's columns the rest alone is needed
+                if (!isc) Q[i * LD + vec - DP] = x[r];
+                else x[r] = 0.0;
+            }
+        }
+        if (isc) length2();
+    }
+    if (on && !isc)
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if (l * R + r >= i) Q[(l * R + r) * LD + vec - DP] = x[r];
     __syncthreads();
     // the basis as used: rounded to FP32, so products with FP32 rows are exact in FP64. Direction i is
     // t = i / 2 of half i % 2, row half * DP/2 + t.
@@ -481,50 +536,56 @@ __global__ __launch_bounds__(BASIS_NT) void prep_basis_kernel(const T *__restric
     }
 }
 
-// One thread per permuted slot: the raw row of the slot-ordered copy, the centred row rotated in FP64 (kept as
-// FP32), its norm, and the maxima per direction. One wave per workgroup: the maxima go through LDS, a lane per
-// direction, then one atomic each.
+// Raw rows of the slot-ordered copy, the centred rows rotated in FP64 (kept as FP32), their norms, and the maxima
+// per direction. 16 slots per workgroup, 16 threads a slot with every 16th direction each: a map has too few
+// neurons for a thread per slot to fill the chip (one wave per 64 slots took 73 us at 1,024 neurons of 40 dims).
+constexpr int ROT_SLOTS = 16, ROT_NT = 256;
 template <int DP, class T>
-__global__ __launch_bounds__(WAVE) void prep_rotate_kernel(const T *__restrict__ w, int mn, int dim, int pblk,
-                                                           const float *__restrict__ centre,
-                                                           const double *__restrict__ basis,
-                                                           const int *__restrict__ perm, T *__restrict__ wslot,
-                                                           float *__restrict__ wrot, double *__restrict__ norms,
-                                                           BmuPlan *__restrict__ plan)
+__global__ __launch_bounds__(ROT_NT) void prep_rotate_kernel(const T *__restrict__ w, int mn, int dim, int pblk,
+                                                             const float *__restrict__ centre,
+                                                             const double *__restrict__ basis,
+                                                             const int *__restrict__ perm, T *__restrict__ wslot,
+                                                             float *__restrict__ wrot, double *__restrict__ norms,
+                                                             BmuPlan *__restrict__ plan)
 {
-    __shared__ float tile[WAVE][DP + 1];
-    const int lane = threadIdx.x;
-    const int p = blockIdx.x * WAVE + lane;
-    const int j = p < pblk * 32 ? perm[p] : -1;
-    double v[DP];
-    double nrm = 0.0;
-#pragma unroll
-    for (int d = 0; d < DP; d++) {
+    __shared__ double bs[DP][DP + 1];
+    __shared__ double v[ROT_SLOTS][DP + 1];
+    __shared__ unsigned int mx[DP];
+    const int tid = threadIdx.x;
+    const int p0 = blockIdx.x * ROT_SLOTS;  // whole blocks of 32 slots: always in range
+    for (int e = tid; e < DP * DP; e += ROT_NT) bs[e / DP][e % DP] = basis[e];
+    for (int e = tid; e < ROT_SLOTS * DP; e += ROT_NT) {
+        const int p = p0 + e / DP, d = e % DP, j = perm[p];
         const T raw = (j >= 0 && d < dim) ? w[(int64_t)j * dim + d] : (T)0;
-        if (p < pblk * 32) wslot[(int64_t)p * DP + d] = raw;
-        v[d] = (j >= 0 && d < dim) ? (double)centred(raw, centre[d]) : 0.0;
-        nrm = fma(v[d], v[d], nrm);
+        wslot[(int64_t)p * DP + d] = raw;
+        v[e / DP][d] = (j >= 0 && d < dim) ? (double)centred(raw, centre[d]) : 0.0;
     }
-#pragma unroll 4
-    for (int i = 0; i < DP; i++) {
-        double r = 0.0;
+    if (tid < DP) mx[tid] = 0u;
+    __syncthreads();
+    const int sl = tid / 16, g = tid % 16;
+    double r[DP / 16];
 #pragma unroll
-        for (int k = 0; k < DP; k++) r = fma(basis[i * DP + k], v[k], r);
-        tile[lane][i] = (float)r;
+    for (int u = 0; u < DP / 16; u++) r[u] = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < DP; k++) {
+        const double x = v[sl][k];
+#pragma unroll
+        for (int u = 0; u < DP / 16; u++) r[u] = fma(bs[g + 16 * u][k], x, r[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < DP / 16; u++) {
+        const int i = g + 16 * u;
+        const float f = (float)r[u];
+        wrot[(int64_t)(p0 + sl) * DP + i] = f;
+        if (fabsf(f) > 0.f) atomicMax(&mx[i], __builtin_bit_cast(unsigned int, fabsf(f)));
+    }
+    if (tid < ROT_SLOTS) {
+        double nrm = 0.0;
+        for (int k = 0; k < DP; k++) nrm = fma(v[tid][k], v[tid][k], nrm);
+        norms[p0 + tid] = perm[p0 + tid] >= 0 ? nrm : __builtin_inf();
     }
     __syncthreads();
-    if (p < pblk * 32) norms[p] = j >= 0 ? nrm : __builtin_inf();
-    constexpr int LPD = WAVE / DP;  // lanes per direction
-    float m = 0.f;
-    const int i = lane % DP;
-#pragma unroll 8
-    for (int r = 0; r < WAVE / LPD; r++) m = fmaxf(m, fabsf(tile[(lane / DP) * (WAVE / LPD) + r][i]));
-    if (m > 0.f) atomicMax(&plan->wmax[i], __builtin_bit_cast(unsigned int, m));
-    // the tile to memory, coalesced
-    for (int e = lane; e < WAVE * DP; e += WAVE) {
-        const int row = e / DP;
-        if (blockIdx.x * WAVE + row < pblk * 32) wrot[(int64_t)blockIdx.x * WAVE * DP + e] = tile[row][e % DP];
-    }
+    if (tid < DP && mx[tid]) atomicMax(&plan->wmax[tid], mx[tid]);
 }
 
 // One neuron's slots of one lane half (values -2 w'' pieces; the norm piece last), and the squares of what the
@@ -613,19 +674,22 @@ __global__ __launch_bounds__(WAVE) void prep_frag_kernel(const T *__restrict__ w
     const int p = blockIdx.x * WAVE + lane;
     if (lane < DP) wm[lane] = __builtin_bit_cast(float, plan->wmax[lane]);
     __syncthreads();
-    float big = lane < DP ? wm[lane] : 0.f, all = big * big;
+    float big = lane < DP ? wm[lane] : 0.f, all = big * big, gap = lane < DP ? plan->step2[lane] : 0.f;
     for (int o = WAVE / 2; o > 0; o >>= 1) {
         big = fmaxf(big, __shfl_xor(big, o, WAVE));
         all += __shfl_xor(all, o, WAVE);
+        gap += __shfl_xor(gap, o, WAVE);
     }
     // the largest value to [2^5, 2^6): norms / 16 stay below 2^15
     const int k = big > 0.f ? min(100, max(-100, 5 - expo(big))) : 0;
-    // the fewest slices whose bound is small against the map, or close to what more of them give. A slice
-    // costs about a quarter of the block loop; a window of 3e-5 of the map, one or two more candidates.
+    // The fewest slices whose bound is small against the map or against the squared distance of neighbouring
+    // neurons, or close to what more of them give. A slice costs about a quarter of the block loop: the first
+    // epoch of a training on 64x64 at D = 16, from random weights far apart, takes 4.9 ms with two and 6.2 ms with
+    // three. A wide window on a smooth map, dozens of candidates: errors of 140,000 rows on 100x90, 506 and 281 us.
     int nk = 2, q3 = 0;
     float e = plan_bound<2, HD>(wm, q3);
-    const float fine = 3e-5f * sqrtf(all);
-    if constexpr (DP > 16) {
+    const float fine = fmaxf(3e-5f * sqrtf(all), gap / (float)mn / (256.f * sqrtf(all)));
+    {
         int q = 0;
         const float e3 = plan_bound<3, HD>(wm, q);
         if (e > fine && e > 2.f * e3) { nk = 3; q3 = q; e = e3; }
@@ -681,12 +745,10 @@ __global__ __launch_bounds__(WAVE) void prep_frag_kernel(const T *__restrict__ w
                 neuron_slots_q<2, HD>(q3, om[h], np, a, lt, nt, rt, ns, rs, nd);
                 put(a, 2);
             }
-            if constexpr (DP > 16) {
-                if (nk == 3) {
-                    f16x8 a[3];
-                    neuron_slots_q<3, HD>(q3, om[h], np, a, lt, nt, rt, ns, rs, nd);
-                    put(a, 3);
-                }
+            if (nk == 3) {
+                f16x8 a[3];
+                neuron_slots_q<3, HD>(q3, om[h], np, a, lt, nt, rt, ns, rs, nd);
+                put(a, 3);
             }
             if constexpr (DP > 32) {
                 if (nk == 5) {
@@ -840,14 +902,11 @@ int prepare_t(somhip_model *M, const T *w, bool rotated)
     hipStream_t st = M->ctx->stream;
     const int slots = M->pblk * 32;
     const dim3 grid((slots + WAVE - 1) / WAVE), block(WAVE);
-    hipLaunchKernelGGL(prep_centre_kernel<T>, dim3(DP), dim3(256), 0, st, w, M->mn, M->dim, DP, M->centre, M->plan);
+    hipLaunchKernelGGL(prep_centre_kernel<T>, dim3(DP), dim3(256), 0, st, w, M->mn, M->n, M->dim, DP, M->centre, M->plan);
     if (rotated) {
-        constexpr size_t lds = basis_lds<DP>();
-        SOM_HIP_TRY(hipFuncSetAttribute((const void *)prep_basis_kernel<DP, T>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((prep_basis_kernel<DP, T>), dim3(1), dim3(BASIS_NT), lds, st, w, M->mn, M->dim, M->centre,
+        hipLaunchKernelGGL((prep_basis_kernel<DP, T>), dim3(1), dim3(BASIS_NT), 0, st, w, M->mn, M->dim, M->centre,
                            M->basis, M->rot, M->plan);
-        hipLaunchKernelGGL((prep_rotate_kernel<DP, T>), grid, block, 0, st, w, M->mn, M->dim, M->pblk, M->centre, M->basis,
+        hipLaunchKernelGGL((prep_rotate_kernel<DP, T>), dim3(slots / ROT_SLOTS), dim3(ROT_NT), 0, st, w, M->mn, M->dim, M->pblk, M->centre, M->basis,
                            M->perm, (T *)M->wslot, M->wrot, M->norms, M->plan);
         hipLaunchKernelGGL((prep_frag_kernel<DP, true, T>), grid, block, 0, st, w, M->mn, M->dim, M->pblk, M->centre,
                            M->perm, (T *)M->wslot, M->wrot, M->norms, (f16x8 *)M->frag_h, f16_nk_limit(M, true), M->plan);
@@ -859,16 +918,21 @@ int prepare_t(somhip_model *M, const T *w, bool rotated)
     return SOMHIP_OK;
 }
 
-// Searches of at least this many (row, neuron) pairs rotate. The rotation costs the basis and one more pass
-// over the weights (40, 100 and 200 us at D = 16, 32 and 64); it saves the wider window of the data's own
-// dimensions at D = 16 and a K slice or two of three to five beyond, a tenth to a third of the search.
-constexpr int64_t rotate_from(int kpad) { return (int64_t)1 << (kpad <= 16 ? 31 : kpad <= 32 ? 30 : 29); }
+// Whether a search of n rows rotates: nearly always. It costs two launches after each change of the weights (20, 40
+// and 75 us at up to 16, 32 and 64 dims), and saves the wider window of the data's own dimensions, which on trained maps
+// fills the candidate lists, and at more than 16 dims K slices. Short searches of small maps do without.
+bool rotate(const somhip_model *M, int64_t n)
+{
+    const int64_t pairs = M->kpad <= 32 ? 1 << 26 : 1 << 25;
+    const int large = M->kpad <= 32 ? 6000 : 4000;
+    return M->mn >= large || n >= pairs / M->mn;
+}
 
 }  // namespace
 
 int somhip_prepare(somhip_model *M, int64_t n)
 {
-    const bool rotated = n >= rotate_from(M->kpad) / M->mn;
+    const bool rotated = rotate(M, n);
     if (M->prepared >= (rotated ? 2 : 1)) return SOMHIP_OK;
     TimerScope ts(M->ctx, TK_PREP);
     int rc;
@@ -892,7 +956,7 @@ int somhip_prepare_f32(somhip_model *M)
     hipStream_t st = M->ctx->stream;
     const dim3 grid((M->nblk * 32 + 255) / 256), block(256);
     if (!M->prepared)  // else the centroid is there, and the plan that this kernel clears is in use (also by a server)
-        hipLaunchKernelGGL(prep_centre_kernel<float>, dim3(M->kpad), dim3(256), 0, st, M->w, M->mn, M->dim, M->kpad,
+        hipLaunchKernelGGL(prep_centre_kernel<float>, dim3(M->kpad), dim3(256), 0, st, M->w, M->mn, M->n, M->dim, M->kpad,
                            M->centre, M->plan);
 #define SOM_PREP(D)                                                                                           \
     hipLaunchKernelGGL(prep_f32_kernel<D>, grid, block, 0, st, M->w, M->mn, M->dim, M->nblk, M->centre,       \
@@ -931,6 +995,7 @@ int64_t somhip_bmu_xmax_rows(int precision, int dpad, int64_t n)
         return (n + per_block - 1) / per_block * BMU_WAVES;
     }
     if (n <= SMALL_ROWS) return (n + NW_SMALL * 32 - 1) / (NW_SMALL * 32) * NW_SMALL;
+    if (n <= MEDIUM_ROWS) return (n + NW_F16 * 32 - 1) / (NW_F16 * 32) * NW_F16;
     return (n + SOM_TILE_ROWS - 1) / SOM_TILE_ROWS * NW_F16;
 }
 
