@@ -546,7 +546,7 @@ int iter_accumulate_t(somhip_accum *A, const T *x, const double *rho, int64_t n,
     if (n == 0) return SOMHIP_OK;
     somhip_ctx *C = M->ctx;
     Workspace &W = A->ws;
-    const int nsplit = somhip_iter_nsplit(n, M->mn);
+    const int nsplit = somhip_iter_nsplit(M, n);
     int rc;
     if ((rc = W.c1.ensure(sizeof(int32_t) * n)) ||
         (rc = A->upd.ensure(sizeof(double) * (size_t)nsplit * M->mn * (M->dim + 1))))
@@ -556,7 +556,7 @@ int iter_accumulate_t(somhip_accum *A, const T *x, const double *rho, int64_t n,
     if ((rc = search(M, x, n, precision, arithmetic, 0, -1, c1, nullptr, nullptr))) return rc;
     TimerScope ts(C, TK_ITER);
     return somhip_launch_iter(C->stream, c1, x, M->dim, M->dpad, rho, n, cur_vector, n_vectors, sigma0,
-                              model_topo<T>(M), M->mn, (double *)A->upd.p, nsplit, A->acc);
+                              model_topo<T>(M), M->mn, M->n, somhip_iter_grid(M), (double *)A->upd.p, nsplit, A->acc);
 }
 
 template <class T>

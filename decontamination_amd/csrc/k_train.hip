@@ -700,14 +700,148 @@ __global__ __launch_bounds__(256) void iter_partial_kernel(const int32_t *__rest
     }
 }
 
-// acc[e] += sum_p part[p][e] (fixed order)
-__global__ void sum_parts_kernel(const double *__restrict__ part, int nsplit, int64_t width, double *__restrict__ acc)
+// The same on the closed-form grids, where exp(-|t_j - t_bmu|^2 / 2 sigma^2) is a product of one factor of the map row
+// (and, on the hexagonal grid, the column's parity) and one of the column: per sample a workgroup of 256 neurons
+// takes (2 rows + columns) exponentials instead of 256, and the sums of h x are FP64 matrix products (16 neurons x 4
+// samples by 4 samples x 16 dims).
+// What bounds it: the FP64 rate, 64 cycles per product of 1,024, with the exponentials and table reads beside them. 100,000
+// samples of 16 dims on 32x32 take 177 us, 447 us with an exponential and 16 conversions per neuron and sample.
+// Four waves of 4 x 16 neurons each. Operand layout: A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k, D[4 r + q][j]
+// in lane j + 16 q, register r.
+template <int DP>
+constexpr int iter_ts() { return DP <= 32 ? 64 : 32; }  // samples per step
+// Map rows that 256 consecutive neurons touch, at most.
+__host__ __device__ constexpr int iter_rows(int mn, int ncol)
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= width) return;
+    const int r = 255 / ncol + 2, all = (mn + ncol - 1) / ncol;
+    return r < all ? r : all;
+}
+template <int DP>
+__host__ __device__ constexpr size_t iter_lds(int mn, int ncol)
+{
+    return sizeof(double) * iter_ts<DP>() * (DP + 2 * iter_rows(mn, ncol) + ncol + 1);
+}
+
+template <int DP, class T>
+__global__ __launch_bounds__(256) void iter_grid_kernel(const int32_t *__restrict__ bmu, const T *__restrict__ x, int dim,
+                                                        const double *__restrict__ rho, int64_t n, int64_t cur,
+                                                        int64_t nvec, T sigma0, const T *__restrict__ topo, int mn,
+                                                        int ncol, int64_t chunk, double *__restrict__ part)
+{
+    typedef double f64x4 __attribute__((ext_vector_type(4)));
+    constexpr int TS = iter_ts<DP>(), NB = DP / 16;
+    extern __shared__ double s_lds[];
+    __shared__ T s_tb[TS * 2];
+    __shared__ double s_inv[TS], s_h0[TS];  // 1 / (2 sigma_i^2); rho_i (rounded to the data type), 0 when left out
+    const int j0 = blockIdx.x * 256, row0 = j0 / ncol;
+    const int nx = 2 * iter_rows(mn, ncol), ne = nx + ncol, es = ne | 1;
+    double *s_x = s_lds;            // [TS][DP]
+    double *s_e = s_x + TS * DP;    // [TS][es]: per sample the factors of (row, column parity), then of the columns
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t ibeg = (int64_t)blockIdx.y * chunk, iend = min(n, ibeg + chunk);
+    // this lane's neuron of each of the wave's four tiles
+    int ex[4], ey[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int j = min(j0 + wave * 64 + t * 16 + (lane & 15), mn - 1), a = j / ncol, b = j - a * ncol;
+        ex[t] = 2 * (a - row0) + (b & 1);
+        ey[t] = nx + b;
+    }
+    f64x4 acc[4][NB];
+    double hs[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        hs[t] = 0.0;
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[t][b] = f64x4{0.0, 0.0, 0.0, 0.0};
+    }
+    for (int64_t i0 = ibeg; i0 < iend; i0 += TS) {
+        __syncthreads();  // the step before has been read
+        if (tid < TS) {
+            const int64_t i = i0 + tid;
+            const int c = i < iend ? bmu[i] : -1;
+            const T r = i < iend && rho ? (T)rho[i] : (T)1;
+            const bool ok = c >= 0 && r > (T)0;
+            s_tb[2 * tid] = ok ? topo[2 * c] : (T)0;
+            s_tb[2 * tid + 1] = ok ? topo[2 * c + 1] : (T)0;
+            double sg = (double)sigma0 * (1.0 / (1.0 + 2.0 * (double)(cur + i) / (double)nvec));
+            if (sg < SOM_FLOAT_EPS) sg = SOM_FLOAT_EPS;
+            s_inv[tid] = 1.0 / (2.0 * sg * sg);
+            s_h0[tid] = ok ? (double)r : 0.0;
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int e = tid; e < TS * DP; e += 256) {
+            // samples left out are zeros: they may hold NaN
+            const int ii = e / DP, k = e % DP;
+            s_x[e] = k < dim && s_h0[ii] > 0.0 ? (double)x[(i0 + ii) * dim + k] : 0.0;
+        }
+        for (int ii = wave; ii < TS; ii += 4) {
+            const T tb0 = s_tb[2 * ii], tb1 = s_tb[2 * ii + 1];
+            const double inv = s_inv[ii];
+            for (int e = lane; e < ne; e += 64) {
+                // coordinate of the row (with the column's parity) or of the column, from the topography itself
+                const int a = min(row0 + e / 2, (mn - 1) / ncol), b = ncol > 1 ? e & 1 : 0;
+                const T d = e < nx ? topo[2 * (a * ncol + b)] - tb0 : topo[2 * (e - nx) + 1] - tb1;
+                const T q = d * d;
+                s_e[ii * es + e] = exp(-(double)q * inv);
+            }
+        }
+        __syncthreads();
+#pragma unroll 2
+        for (int v0 = 0; v0 < TS; v0 += 4) {
+            const int ii = v0 + (lane >> 4);
+            const double h0 = s_h0[ii];
+            double bx[NB];
+#pragma unroll
+            for (int b = 0; b < NB; b++) bx[b] = s_x[ii * DP + 16 * b + (lane & 15)];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const double h = h0 * (s_e[ii * es + ex[t]] * s_e[ii * es + ey[t]]);
+                hs[t] += h;
+#pragma unroll
+                for (int b = 0; b < NB; b++) acc[t][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(h, bx[b], acc[t][b], 0, 0, 0);
+            }
+        }
+    }
+    const int nv = dim + 1;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int jt = j0 + wave * 64 + t * 16;
+        hs[t] += __shfl_xor(hs[t], 16);
+        hs[t] += __shfl_xor(hs[t], 32);
+        if (lane < 16 && jt + lane < mn) part[((int64_t)blockIdx.y * mn + jt + lane) * nv + dim] = hs[t];
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int j = jt + 4 * r + (lane >> 4), k = 16 * b + (lane & 15);
+                if (j < mn && k < dim) part[((int64_t)blockIdx.y * mn + j) * nv + k] = acc[t][b][r];
+            }
+    }
+}
+
+// acc[e] += sum_p part[p][e]: 8 threads an element, every eighth part each, joined in fixed order (one thread an element, a
+// serial chain of loads on few CUs, took 63 us for 256 parts of 17,408 sums).
+constexpr int SP_LANES = 8;
+__global__ __launch_bounds__(256) void sum_parts_kernel(const double *__restrict__ part, int nsplit, int64_t width,
+                                                        double *__restrict__ acc)
+{
+    constexpr int EL = 256 / SP_LANES;
+    __shared__ double red[SP_LANES][EL];
+    const int64_t e = (int64_t)blockIdx.x * EL + threadIdx.x % EL;
+    const int q = threadIdx.x / EL;
     double s = 0.0;
-    for (int p = 0; p < nsplit; p++) s += part[(int64_t)p * width + e];
-    acc[e] += s;
+    if (e < width) {
+#pragma unroll 8
+        for (int p = q; p < nsplit; p += SP_LANES) s += part[(int64_t)p * width + e];
+    }
+    red[q][threadIdx.x % EL] = s;
+    __syncthreads();
+    if (q == 0 && e < width) {
+        for (int u = 1; u < SP_LANES; u++) s += red[u][threadIdx.x];
+        acc[e] += s;
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -967,8 +1101,25 @@ int somhip_launch_divide(hipStream_t st, const double *acc, int mn, int dim, T *
     return SOMHIP_OK;
 }
 
-int somhip_iter_nsplit(int64_t n, int mn)
+// Whether the vector-count sums take the grid form: its tables fit 64 KB of LDS (up to about 70 columns).
+static size_t iter_grid_lds(int dpad, int mn, int ncol)
 {
+    return dpad == 16 ? iter_lds<16>(mn, ncol) : dpad == 32 ? iter_lds<32>(mn, ncol)
+                                             : dpad == 48 ? iter_lds<48>(mn, ncol) : iter_lds<64>(mn, ncol);
+}
+bool somhip_iter_grid(const somhip_model *M)
+{
+    return M->separable && iter_grid_lds(M->dpad, M->mn, M->n) <= 62 * 1024;
+}
+
+int somhip_iter_nsplit(const somhip_model *M, int64_t n)
+{
+    const int mn = M->mn;
+    if (somhip_iter_grid(M)) {
+        // three workgroups per CU, of at least two steps each
+        const int64_t tiles = (mn + 255) / 256;
+        return (int)std::max<int64_t>(1, std::min<int64_t>((n + 127) / 128, 768 / tiles));
+    }
     int64_t s = std::max<int64_t>(1, (int64_t)262144 / std::max(mn, 1));
     s = std::min<int64_t>(s, std::max<int64_t>(1, n / 64));
     return (int)std::min<int64_t>(s, 4096);
@@ -976,23 +1127,33 @@ int somhip_iter_nsplit(int64_t n, int mn)
 
 template <class T>
 int somhip_launch_iter(hipStream_t st, const int32_t *bmu, const T *x, int dim, int dpad, const double *rho,
-                       int64_t n, int64_t cur, int64_t nvec, T sigma0, const T *topo, int mn, double *part,
-                       int nsplit, double *acc)
+                       int64_t n, int64_t cur, int64_t nvec, T sigma0, const T *topo, int mn, int ncol, bool grid,
+                       double *part, int nsplit, double *acc)
 {
     if (n <= 0) return SOMHIP_OK;
     const int64_t chunk = (n + nsplit - 1) / nsplit;
     dim3 g((mn + 255) / 256, nsplit), b(256);
 #define SOM_IT(D) hipLaunchKernelGGL((iter_partial_kernel<D, T>), g, b, 0, st, bmu, x, dim, rho, n, cur, nvec, sigma0, topo, mn, chunk, part)
+#define SOM_IG(D)                                                                                                    \
+    hipLaunchKernelGGL((iter_grid_kernel<D, T>), g, b, iter_lds<D>(mn, ncol), st, bmu, x, dim, rho, n, cur, nvec,   \
+                       sigma0, topo, mn, ncol, chunk, part)
+#define SOM_ITG(D)                                                                                                   \
+    do {                                                                                                             \
+        if (grid) SOM_IG(D); else SOM_IT(D);                                                                         \
+    } while (0)
     switch (dpad) {
-        case 16: SOM_IT(16); break;
-        case 32: SOM_IT(32); break;
-        case 48: SOM_IT(48); break;
-        default: SOM_IT(64); break;
+        case 16: SOM_ITG(16); break;
+        case 32: SOM_ITG(32); break;
+        case 48: SOM_ITG(48); break;
+        default: SOM_ITG(64); break;
     }
+#undef SOM_ITG
+#undef SOM_IG
 #undef SOM_IT
     SOM_HIP_TRY(hipGetLastError());
     const int64_t width = (int64_t)mn * (dim + 1);
-    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((width + 255) / 256)), dim3(256), 0, st, part, nsplit, width,
+    constexpr int EL = 256 / SP_LANES;
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((width + EL - 1) / EL)), dim3(256), 0, st, part, nsplit, width,
                        acc);
     SOM_HIP_TRY(hipGetLastError());
     return SOMHIP_OK;
@@ -1028,7 +1189,7 @@ int somhip_launch_errors(hipStream_t st, const int32_t *c1, const int32_t *c2, c
                                                    double, double *, T *, T *);                                 \
     template int somhip_launch_divide<T>(hipStream_t, const double *, int, int, T *, T *);                      \
     template int somhip_launch_iter<T>(hipStream_t, const int32_t *, const T *, int, int, const double *,       \
-                                       int64_t, int64_t, int64_t, T, const T *, int, double *, int, double *);  \
+                                       int64_t, int64_t, int64_t, T, const T *, int, int, bool, double *, int, double *);  \
     template int somhip_launch_errors<T>(hipStream_t, const int32_t *, const int32_t *, const double *,         \
                                          const double *, int64_t, const T *, double, double *, int, double *);
 SOM_TRAIN_LAUNCHERS(float)

@@ -34,11 +34,12 @@ int somhip_launch_update_separable(hipStream_t st, const double *S, const R *top
                                    double sigma, double *T, R *w, R *hist);
 template <class T>
 int somhip_launch_divide(hipStream_t st, const double *acc, int mn, int dim, T *w, T *hist);
-int somhip_iter_nsplit(int64_t n, int mn);
+bool somhip_iter_grid(const somhip_model *M);
+int somhip_iter_nsplit(const somhip_model *M, int64_t n);
 template <class T>
 int somhip_launch_iter(hipStream_t st, const int32_t *bmu, const T *x, int dim, int dpad, const double *rho,
-                       int64_t n, int64_t cur, int64_t nvec, T sigma0, const T *topo, int mn, double *part,
-                       int nsplit, double *acc);
+                       int64_t n, int64_t cur, int64_t nvec, T sigma0, const T *topo, int mn, int ncol, bool grid,
+                       double *part, int nsplit, double *acc);
 int somhip_errors_nparts(int64_t n);
 template <class T>
 int somhip_launch_errors(hipStream_t st, const int32_t *c1, const int32_t *c2, const double *d1, const double *rho,
