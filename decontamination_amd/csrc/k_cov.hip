@@ -2,11 +2,14 @@
 // _update_welford_cov_sums :30-84 and _finalize_welford_cov :90-119), the pass that initialises a
 // SOM_PCA.
 //
-// The reference runs Welford's update sample by sample on one CPU thread. Here one chunk takes two
-// HBM-bound streaming passes with fixed-order reductions (deterministic):
-//   pass 1: W = sum w and sum w x over the valid rows, mean = sum w x / W;
-//   pass 2: the corrected two-pass sums on d = x - mean, S = sum w d d^T and c = sum w d, from which
-//           the host forms M2 = S - c c^T / W and mean + c / W.
+// The reference runs Welford's update sample by sample on one CPU thread. Here one chunk takes one
+// HBM-bound streaming pass with fixed-order reductions (deterministic), after a look at a sample:
+//   pass 1: sum w and sum w x over the valid rows of a sample spread over the chunk (short chunks: all rows), whose
+//           mean is the shift;
+//   pass 2: on d = x - shift, W = sum w, S = sum w d d^T and c = sum w d, from which the host forms
+//           M2 = S - c c^T / W and the mean, shift + c / W.
+// The correction cancels (shift - mean)^2 against S: where it is more than 1/64 of a column's variance, pass 2 runs
+// again with the mean that it found as the shift, which is the corrected two-pass form.
 // A row is valid when its weight is finite and > 0 and all its values are finite (the reference's
 // rule). Chunks are merged on the host with Chan's update.
 //
@@ -68,17 +71,17 @@ __device__ __forceinline__ double check_row(const T (&raw)[NBLK], double w, int6
     return w;
 }
 
-// pass 1: per-workgroup partials [sum w, sum w x_col (col < 16*NBLK)]
+// pass 1: per-workgroup partials [sum w, sum w x_col (col < 16*NBLK)] over the first `take` rows of each range
 template <typename T, int NBLK>
 __global__ __launch_bounds__(COV_NT) void cov_pass1_kernel(const T *x, const double *rho, int64_t n, int dim,
-                                                           int64_t rows_per_wg, double *part)
+                                                           int64_t rows_per_wg, int64_t take, double *part)
 {
     constexpr int DP = 16 * NBLK;
     __shared__ double red[COV_NT / 64][DP + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 15, k = lane >> 4;
     const int64_t r0 = (int64_t)blockIdx.x * rows_per_wg;
-    const int64_t r1 = min(n, r0 + rows_per_wg);
+    const int64_t r1 = min(n, r0 + min(rows_per_wg, take));
     double sw = 0.0, sx[NBLK];
 #pragma unroll
     for (int b = 0; b < NBLK; b++) sx[b] = 0.0;
@@ -120,19 +123,22 @@ __global__ __launch_bounds__(COV_NT) void cov_pass1_kernel(const T *x, const dou
     }
 }
 
-// pass 2: per-workgroup partials [S tiles (T tiles x 256, D[i][j] at 16 i + j), c (16*NBLK)]
+// pass 2: per-workgroup partials [S tiles (T tiles x 256, D[i][j] at 16 i + j), c (16*NBLK), W].
+// Bound by issue: an FP64 product and about ten FP64 instructions per 4 rows beside 2.6 TB/s of loads. A step of 8 quads
+// whose rows are all valid, tested with one ballot, needs no zeroing: 351 us for 12.6 M weighted rows of 16 dims, 361 us
+// with a ballot per quad. Reading all rows for the shift too took another 262 us, a sample of them 14 us.
 template <typename T, int NBLK>
 __global__ __launch_bounds__(COV_NT) void cov_pass2_kernel(const T *x, const double *rho, int64_t n, int dim,
                                                            int64_t rows_per_wg, const double *sums, double *part)
 {
     constexpr int DP = 16 * NBLK;
     constexpr int NT = NBLK * (NBLK + 1) / 2;  // upper-triangle 16x16 tiles
-    constexpr int OUT = NT * 256 + DP;
+    constexpr int OUT = NT * 256 + DP + 1;
     __shared__ double red[COV_NT / 64][OUT];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 15, k = lane >> 4;
     const double W = sums[0];
-    double mean[NBLK];
+    double sw = 0.0, mean[NBLK];
 #pragma unroll
     for (int b = 0; b < NBLK; b++) {
         const int col = 16 * b + j;
@@ -148,18 +154,36 @@ __global__ __launch_bounds__(COV_NT) void cov_pass2_kernel(const T *x, const dou
     for (int b = 0; b < NBLK; b++) cs[b] = 0.0;
     for (int64_t q0 = r0 + 4 * wave; q0 < r1; q0 += 4 * 4 * COV_UNROLL) {
         T raw[COV_UNROLL][NBLK];
-        double v[COV_UNROLL][NBLK], w[COV_UNROLL];
+        double w[COV_UNROLL];
         // all loads of the step first, then the checks (their ballots wait for the data)
 #pragma unroll
         for (int u = 0; u < COV_UNROLL; u++) load_row<T, NBLK>(x, rho, q0 + 16 * u + k, r1, dim, j, raw[u], w[u]);
+        bool fine = true;  // columns past dim repeat the last one
 #pragma unroll
-        for (int u = 0; u < COV_UNROLL; u++) w[u] = check_row<T, NBLK>(raw[u], w[u], q0 + 16 * u + k, r1, dim, j, k, v[u]);
+        for (int u = 0; u < COV_UNROLL; u++) {
+            if (rho) fine = fine && __builtin_isfinite(w[u]) && w[u] > 0.0;
+#pragma unroll
+            for (int b = 0; b < NBLK; b++) fine = fine && finite_val(raw[u][b]);
+        }
+        const bool all = q0 + 16 * (COV_UNROLL - 1) + 4 <= r1 && __ballot(!fine) == 0ull;  // uniform
+        if (!all) {
+            // invalid rows become rows of the shift with weight 0
+#pragma unroll
+            for (int u = 0; u < COV_UNROLL; u++) {
+                double v[NBLK];
+                w[u] = check_row<T, NBLK>(raw[u], w[u], q0 + 16 * u + k, r1, dim, j, k, v);
+#pragma unroll
+                for (int b = 0; b < NBLK; b++) raw[u][b] = w[u] > 0.0 ? raw[u][b] : (T)0;
+            }
+        }
 #pragma unroll
         for (int u = 0; u < COV_UNROLL; u++) {
             double d[NBLK], wd[NBLK];
+            sw += w[u];
 #pragma unroll
             for (int b = 0; b < NBLK; b++) {
-                d[b] = w[u] > 0.0 ? v[u][b] - mean[b] : 0.0;
+                // columns past dim: their tile entries are not read
+                d[b] = (double)raw[u][b] - mean[b];
                 wd[b] = w[u] * d[b];
                 cs[b] += wd[b];
             }
@@ -183,6 +207,9 @@ __global__ __launch_bounds__(COV_NT) void cov_pass2_kernel(const T *x, const dou
     if (lane < 16)
 #pragma unroll
         for (int b = 0; b < NBLK; b++) red[wave][NT * 256 + 16 * b + j] = cs[b];
+    sw += __shfl_xor(sw, 16);
+    sw += __shfl_xor(sw, 32);
+    if (lane == 0) red[wave][OUT - 1] = sw;
     __syncthreads();
     for (int e = threadIdx.x; e < OUT; e += COV_NT) {
         double s = 0.0;
@@ -208,7 +235,7 @@ template <typename T, int NBLK>
 int cov_launch(somhip_ctx *C, const T *x, const double *rho, int64_t n, int dim, double *out_host)
 {
     constexpr int NT = NBLK * (NBLK + 1) / 2;
-    constexpr int OUT = NT * 256 + 16 * NBLK;
+    constexpr int OUT = NT * 256 + 16 * NBLK + 1;
     hipStream_t st = C->stream;
     // one round of resident workgroups, each a contiguous run of whole row quads
     static int per_cu = 0;
@@ -229,25 +256,44 @@ int cov_launch(somhip_ctx *C, const T *x, const double *rho, int64_t n, int dim,
     double *part = (double *)Wk.part.p;
     double *sums = (double *)Wk.maps.p;
     double *tiles = sums + dim + 1;
-    hipLaunchKernelGGL((cov_pass1_kernel<T, NBLK>), dim3(G), dim3(COV_NT), 0, st, x, rho, n, dim, rows_per_wg, part);
+    // 128 rows of each of a thousand ranges place the shift within a few thousandths of a deviation
+    const int64_t take = n <= 262144 ? rows_per_wg : 128;
+    hipLaunchKernelGGL((cov_pass1_kernel<T, NBLK>), dim3(G), dim3(COV_NT), 0, st, x, rho, n, dim, rows_per_wg, take, part);
     SOM_HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(cov_reduce_kernel, dim3(dim + 1), dim3(256), 0, st, part, G, dim + 1, sums);
     SOM_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL((cov_pass2_kernel<T, NBLK>), dim3(G), dim3(COV_NT), 0, st, x, rho, n, dim, rows_per_wg, sums,
-                       part);
-    SOM_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(cov_reduce_kernel, dim3(OUT), dim3(256), 0, st, part, G, OUT, tiles);
-    SOM_HIP_TRY(hipGetLastError());
     std::vector<double> h((size_t)dim + 1 + OUT);
-    SOM_HIP_TRY(hipMemcpyAsync(h.data(), sums, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
-    SOM_HIP_TRY(hipStreamSynchronize(st));
-    // W, mean (the division pass 2 used), then M2 = S - c c^T / W and mean += c / W
-    const double W = h[0];
     const double *S = h.data() + dim + 1;
     const double *c = S + NT * 256;
+    double W = 0.0;
+    for (int pass = 0;; pass++) {
+        hipLaunchKernelGGL((cov_pass2_kernel<T, NBLK>), dim3(G), dim3(COV_NT), 0, st, x, rho, n, dim, rows_per_wg, sums,
+                           part);
+        SOM_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(cov_reduce_kernel, dim3(OUT), dim3(256), 0, st, part, G, OUT, tiles);
+        SOM_HIP_TRY(hipGetLastError());
+        SOM_HIP_TRY(hipMemcpyAsync(h.data(), sums, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
+        SOM_HIP_TRY(hipStreamSynchronize(st));
+        W = c[16 * NBLK];
+        // the shift's distance to the mean, against the deviation about the mean
+        bool near = true;
+        for (int a = 0; a < dim; a++) {
+            const int t = (a / 16) * NBLK - (a / 16) * (a / 16 - 1) / 2;  // tile (a / 16, a / 16)
+            const double off2 = c[a] * c[a] / W, var = S[t * 256 + 17 * (a % 16)] - off2;
+            near = near && (off2 == 0.0 || off2 <= var / 64.0);
+        }
+        if (pass == 1 || near || !(W > 0.0)) break;
+        // the mean found so far (sums over W, as the kernel divides them)
+        std::vector<double> again((size_t)dim + 1);
+        again[0] = W;
+        for (int a = 0; a < dim; a++) again[1 + a] = ((h[0] > 0.0 ? h[1 + a] / h[0] : 0.0) + c[a] / W) * W;
+        SOM_HIP_TRY(hipMemcpyAsync(sums, again.data(), sizeof(double) * again.size(), hipMemcpyHostToDevice, st));
+        SOM_HIP_TRY(hipStreamSynchronize(st));
+    }
+    // W, the shift (the division pass 2 used), then M2 = S - c c^T / W and the mean, shift + c / W
     out_host[0] = W;
     double *mean = out_host + 1, *m2 = out_host + 1 + dim;
-    for (int a = 0; a < dim; a++) mean[a] = W > 0.0 ? h[1 + a] / W : 0.0;
+    for (int a = 0; a < dim; a++) mean[a] = W > 0.0 && h[0] > 0.0 ? h[1 + a] / h[0] : 0.0;
     for (int a = 0; a < dim; a++)
         for (int b = 0; b < dim; b++) {
             const int lo = std::min(a, b), hi = std::max(a, b);
