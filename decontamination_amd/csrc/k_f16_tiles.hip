@@ -3,19 +3,20 @@
 
 namespace {
 
-// Serving form: one workgroup per tile; tiles of different requests and models share one launch.
-template <int DP, int G, int MODE, bool NEED_C2>
-__global__ __launch_bounds__(NW_F16 * WAVE, 4) void bmu_f16_tiles_kernel(const BmuModelDev *__restrict__ models,
+// Serving form: one workgroup per tile; tiles of different requests and models share one launch. NW waves of G groups.
+template <int DP, int NW, int G, int MODE, bool NEED_C2>
+__global__ __launch_bounds__(NW * WAVE, 4) void bmu_f16_tiles_kernel(const BmuModelDev *__restrict__ models,
                                                                          const BmuTile *__restrict__ tiles,
                                                                          int64_t *__restrict__ fb_list,
                                                                          unsigned int *__restrict__ fb_count)
 {
-    __shared__ F16Smem<DP / 16, NW_F16, G> sm;
+    static_assert(NW * G * 32 == SOM_TILE_ROWS, "a tile per workgroup");
+    __shared__ F16Smem<DP / 16, NW, G> sm;
     const BmuTile T = tiles[blockIdx.x];
     if (T.n <= 0) return;  // uniform over the workgroup
     const BmuModelDev Md = models[T.model];
     // the descriptors' pointers are generic to the compiler: global_* accesses instead of flat ones
-    bmu_f16_run<DP, f16_max_nk(DP), NW_F16, G, MODE, NEED_C2, true, float>(Md, T.x, T.n, T.row0, T.default_index, T.c1, T.c2, T.d1, fb_list,
+    bmu_f16_run<DP, f16_max_nk(DP), NW, G, MODE, NEED_C2, true, float>(Md, T.x, T.n, T.row0, T.default_index, T.c1, T.c2, T.d1, fb_list,
                                                    fb_count, (int64_t)blockIdx.x << FB_TILE_SHIFT, sm, nullptr, nullptr);
 }
 
@@ -43,6 +44,8 @@ __global__ __launch_bounds__(FB_THREADS) void bmu_exact_tiles_kernel(const BmuMo
     }
 }
 
+constexpr int TILES_FEW = 256;  // one tile per CU
+
 }  // namespace
 
 int somhip_launch_bmu_tiles(hipStream_t st, int dpad, int arithmetic, int need_c2, const BmuModelDev *models,
@@ -53,12 +56,20 @@ int somhip_launch_bmu_tiles(hipStream_t st, int dpad, int arithmetic, int need_c
         somhip_set_error("serving supports dim <= 32");
         return SOMHIP_ERR_UNSUPPORTED;
     }
-    dim3 g((unsigned)grid), b(NW_F16 * WAVE);
+    // Launches that leave CUs with one tile take it in 16 waves of one group, which hide each other's latency: 250,000 rows of requests to a
+    // 64x64 map of 32 dims and a 32x32 one took 172 and 55 us a launch in 8 waves of two groups, 140 and 48 us so.
+    // Fuller ones keep 8 waves of two groups, which read each fragment once for both.
+    const bool few = grid <= TILES_FEW;
+    dim3 g((unsigned)grid);
     const int fb_grid = std::max(1, std::min(grid, 1024));
 #define SOM_TL(D, MO, C)                                                                                  \
     do {                                                                                                  \
-        hipLaunchKernelGGL((bmu_f16_tiles_kernel<D, G_F16, MO, C>), g, b, 0, st, models, tiles, fb_list, \
-                           fb_count);                                                                    \
+        if (few)                                                                                          \
+            hipLaunchKernelGGL((bmu_f16_tiles_kernel<D, 2 * NW_F16, 1, MO, C>), g, dim3(2 * NW_F16 * WAVE), 0, st, models, \
+                               tiles, fb_list, fb_count);                                                 \
+        else                                                                                              \
+            hipLaunchKernelGGL((bmu_f16_tiles_kernel<D, NW_F16, G_F16, MO, C>), g, dim3(NW_F16 * WAVE), 0, st, models, \
+                               tiles, fb_list, fb_count);                                                 \
         hipLaunchKernelGGL((bmu_exact_tiles_kernel<D, MO>), dim3(fb_grid), dim3(256), 0, st, models,       \
                            tiles, fb_list, fb_count);                                                    \
     } while (0)
