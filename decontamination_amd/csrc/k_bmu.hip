@@ -685,10 +685,12 @@ __global__ __launch_bounds__(WAVE) void prep_frag_kernel(const T *__restrict__ w
     // The fewest slices whose bound is small against the map or against the squared distance of neighbouring
     // neurons, or close to what more of them give. A slice costs about a quarter of the block loop: the first
     // epoch of a training on 64x64 at D = 16, from random weights far apart, takes 4.9 ms with two and 6.2 ms with
-    // three. A wide window on a smooth map, dozens of candidates: errors of 140,000 rows on 100x90, 506 and 281 us.
+    // three. A wide window on a smooth map, dozens of candidates: errors of 140,000 rows on 100x90, 506 and 281 us. The
+    // sixth lies between trained maps where two slices are better (winners of 1,000,003 rows on 64x64 at D = 13, a
+    // ninth: 405 and 470 us) and where three are (errors of 1,000,000 rows on 40x50 at D = 32, two fifths: 790 and 570).
     int nk = 2, q3 = 0;
     float e = plan_bound<2, HD>(wm, q3);
-    const float fine = fmaxf(3e-5f * sqrtf(all), gap / (float)mn / (256.f * sqrtf(all)));
+    const float fine = fmaxf(3e-5f * sqrtf(all), gap / (float)mn / (6.f * sqrtf(all)));
     {
         int q = 0;
         const float e3 = plan_bound<3, HD>(wm, q);
