@@ -264,7 +264,7 @@ def pipeline_bench(ctx, X, x_dev, W, m, arith, steps=20):
     return {
         "covariance": {"ms": round(1e3 * t_cov, 4), "rows_per_s": round(N / t_cov, 1),
                        "algorithmic_GB_per_s": round(algo_cov / t_cov / 1e9, 1),
-                       "note": f"weighted covariance of the {N}x{dim} footprint (SOM_PCA init), 2 passes over X, "
+                       "note": f"weighted covariance of the {N}x{dim} footprint (SOM_PCA init), a sample and a pass over X, "
                                "wall clock per call incl. the 2 KB result copy",
                        "cpu_baseline": {"value": round(cpu_cov, 1), "unit": "rows/s", "cores": 1, "kind": "port",
                                         "sample": f"oracle Welford loop (sequential, as the reference's) on the "
